@@ -6,6 +6,7 @@
 
 #include <algorithm>
 
+#include "deq.hpp"
 #include "kernels.hpp"
 
 namespace rehip {
@@ -680,161 +681,229 @@ size_t attention_work_floats(int rows, int heads, int hd, int max_seq) {
   return (size_t)rows * heads * nsp * (hd + 2);
 }
 
-// Many rows, head size 64 (prefill): f32 MFMA flash attention. A workgroup owns 32 query
-// vectors of one kv head (vector g = row * grp + head-in-group, so a block may cut across
-// rows) and its four waves split the cache into 32-key blocks (wave w takes blocks w, w+4, ..).
+// Many rows, head sizes 32 / 64 / 96 / 128 (prefill): f32 MFMA flash attention. A workgroup owns 32
+// query vectors of one kv head (vector g = row * grp + head-in-group, so a block may cut across
+// rows) and its eight waves split the cache into 32-key blocks (wave w takes blocks w, w + 8, ..).
 // Per key block, in v_mfma_f32_32x32x2_f32 layout with lane l = (half h = l/32, column l%32):
-//   S^T[key][vec] = K Q^T: A = K[key l%32][dim 32h + s], B = Q[vec l%32][dim 32h + s],
-//     s = 0..31; register i of the result is key 8(i/4) + 4h + i%4 of vector l%32;
+//   S^T[key][vec] = K Q^T: A = K[key l%32][dim], B = Q[vec l%32][dim], the lane's dims of step
+//     (t, e) being 8t + 4h + e (any order serves the sum; this one lets the two halves of a row
+//     read 32 contiguous bytes); register i of the result is key 8(i/4) + 4h + i%4 of vector l%32;
 //   online softmax per vector (running max m, rescale of earlier terms by exp(m_old - m_new));
 //   O^T[dim][vec] += V^T P^T: step s takes the key held in result register s, so the B operand
 //     is that register and A = V[that key][dim l%32 + 32 nb].
-// The four waves' (m, sum, O) are combined in LDS in wave order. K and V of the next key block
-// are loaded while the current one is in the MFMAs. Row blocks run longest-first.
-constexpr int kAttnMfmaVecs = 32;
+// The waves' (m, sum, O) are combined in LDS in wave order. Row blocks run longest-first, kv heads
+// interleaved (an XCD serves as few kv heads as it can, so their K/V stay in its L2).
+// Bound by the f32 matrix cores (64 cycles per MFMA). V and the next block's K are loaded ahead of the
+// softmax, one or a few thousand cycles before their use. The queries are
+// read from LDS, not held in registers: K (HD/2 registers), V (HD/2) and O (HD/2) then fit two
+// waves per SIMD at HD = 128, so one wave's softmax runs under the other's MFMAs. Eight waves on one
+// block of vectors instead of two workgroups of four: the longest rows finish in half the time.
+// Measured: 1000 rows at position 1048, 32 / 4 heads of 128: 266 us (60 % of the MFMA rate; 2549 us on
+// the per-(head, row) kernel), 961 rows, 14 / 2 heads of 64: 32.8 us (37.2 on four waves per block).
+constexpr int kAttnMfmaVecs = 32, kAttnMfmaWaves = 8;
 
 __device__ __forceinline__ int attn_key_of(int i, int h) { return 8 * (i >> 2) + 4 * h + (i & 3); }
 
-__global__ __launch_bounds__(256) void attention_mfma_kernel(const float* __restrict__ q, const float* __restrict__ kc,
-                                                             const float* __restrict__ vc, int rows, int heads,
-                                                             int kv_heads, int max_seq, const int* __restrict__ pos,
-                                                             float* __restrict__ ctx) {
-  constexpr int HD = 64;
-  typedef float f32x16 __attribute__((ext_vector_type(16)));
-  __shared__ __attribute__((aligned(16))) float Os[4][kAttnMfmaVecs][HD + 4];
-  __shared__ float Ms[4][kAttnMfmaVecs], Ls[4][kAttnMfmaVecs];
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+// scores of a 32 x 32 block over the dims of steps T0 .. T0 + N - 1 (8 dims each): a chain of four
+// MFMAs per step, the steps added as a tree. One chain over all of HD = 128 rounds 64 times at
+// the size of the whole sum, and its scores' error (and the output's: 1.0e-6 against 64 bits on
+// 1000 x 1548 keys, 3.4e-7 so) was three times the vector kernel's.
+template <int T0, int N, int K>
+__device__ __forceinline__ f32x16 attn_scores(const float (&kd)[K], const float* qr) {
+  if constexpr (N > 1) {
+    const f32x16 a = attn_scores<T0, N / 2>(kd, qr);
+    f32x16 s = a + attn_scores<T0 + N / 2, N - N / 2>(kd, qr);
+    asm volatile("" : "+v"(s));          // added here: gathered at the end, the parts do not fit the registers
+    return s;
+  } else {
+    const float4 x = *reinterpret_cast<const float4*>(qr + 8 * T0);
+    f32x16 s = {};
+    s = __builtin_amdgcn_mfma_f32_32x32x2f32(kd[4 * T0], x.x, s, 0, 0, 0);
+    s = __builtin_amdgcn_mfma_f32_32x32x2f32(kd[4 * T0 + 1], x.y, s, 0, 0, 0);
+    s = __builtin_amdgcn_mfma_f32_32x32x2f32(kd[4 * T0 + 2], x.z, s, 0, 0, 0);
+    s = __builtin_amdgcn_mfma_f32_32x32x2f32(kd[4 * T0 + 3], x.w, s, 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    return s;
+  }
+}
+
+template <int HD>
+__global__ __launch_bounds__(64 * kAttnMfmaWaves) void attention_mfma_kernel(
+    const float* __restrict__ q, const float* __restrict__ kc, const float* __restrict__ vc, int rows, int heads,
+    int kv_heads, int max_seq, const int* __restrict__ pos, float* __restrict__ ctx) {
+  constexpr int NB = HD / 32, NT = HD / 8, LD = HD + 4, W = kAttnMfmaWaves;
+  __shared__ __attribute__((aligned(16))) float Qs[kAttnMfmaVecs][LD];
+  __shared__ __attribute__((aligned(16))) float Os[W][kAttnMfmaVecs][LD];
+  __shared__ float Ms[W][kAttnMfmaVecs], Ls[W][kAttnMfmaVecs];
   const int grp = heads / kv_heads;
-  const int blk = gridDim.x - 1 - blockIdx.x, kvh = blockIdx.y;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int nblk = gridDim.x / kv_heads;
+  const int kvh = blockIdx.x % kv_heads, blk = nblk - 1 - blockIdx.x / kv_heads;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int vl = lane & 31, h = lane >> 5;
   const int kv_dim = kv_heads * HD;
   const int p0 = *pos;
   const int g0 = blk * kAttnMfmaVecs;
   const int r_last = min((g0 + kAttnMfmaVecs - 1) / grp, rows - 1);
-  const int jmax = min(p0 + r_last, max_seq - 1);
+  const int jmax = max(min(p0 + r_last, max_seq - 1), 0);
   const int nkb = jmax / 32 + 1;
-  // this lane's query vector
-  const int g = g0 + vl, r = g / grp, head = kvh * grp + g % grp;
-  const bool valid = r < rows;
-  const int limit = valid ? min(p0 + r, max_seq - 1) : -1;
-  float qb[32];
-  {
-    const float* qr = q + ((size_t)(valid ? r : 0) * heads + (valid ? head : 0)) * HD + 32 * h;
+  // last key this lane's query vector sees (none for a vector past the last row)
+  const int r = (g0 + vl) / grp;
+  const int limit = r < rows ? max(min(p0 + r, max_seq - 1), 0) : -1;
+  const int lim_first = max(min(p0 + g0 / grp, max_seq - 1), 0);   // of the block's first vector
+  // one per-lane offset plus a scalar row offset; the resources end with the last visible row, so
+  // rows past it are never read (zeros, which no vector sees)
+  const uint32_t row_b = (uint32_t)kv_dim * 4u, cache_b = (uint32_t)jmax * row_b + HD * 4u;
+  const __amdgpu_buffer_rsrc_t kr = make_rsrc(kc + (size_t)kvh * HD, cache_b);
+  const __amdgpu_buffer_rsrc_t vr = make_rsrc(vc + (size_t)kvh * HD, cache_b);
+  const int koff = (int)((uint32_t)vl * row_b + 16u * h), voff = (int)(4u * h * row_b + 4u * vl);
+  float kd[4 * NT], vd[NB][16];
+  auto load_k = [&](int kbi) {
 #pragma unroll
-    for (int t = 0; t < 8; ++t) {
-      const float4 x = valid ? *reinterpret_cast<const float4*>(qr + 4 * t) : make_float4(0.f, 0.f, 0.f, 0.f);
-      qb[4 * t] = x.x;
-      qb[4 * t + 1] = x.y;
-      qb[4 * t + 2] = x.z;
-      qb[4 * t + 3] = x.w;
-    }
-  }
-  const float scale = 1.0f / sqrtf((float)HD);
-  const float* kb = kc + (size_t)kvh * HD;
-  const float* vb = vc + (size_t)kvh * HD;
-  auto load = [&](int kbi, float (&kd)[32], float (&vd)[2][16]) {
-    const float* kr = kb + (size_t)min(32 * kbi + vl, jmax) * kv_dim + 32 * h;
+    for (int t = 0; t < NT; ++t) {
+      const i32x4_t x = __builtin_amdgcn_raw_buffer_load_b128(kr, koff + 32 * t, (int)(32u * kbi * row_b), 0);
 #pragma unroll
-    for (int t = 0; t < 8; ++t) {
-      const float4 x = *reinterpret_cast<const float4*>(kr + 4 * t);
-      kd[4 * t] = x.x;
-      kd[4 * t + 1] = x.y;
-      kd[4 * t + 2] = x.z;
-      kd[4 * t + 3] = x.w;
-    }
-#pragma unroll
-    for (int s = 0; s < 16; ++s) {
-      const float* vr = vb + (size_t)min(32 * kbi + attn_key_of(s, h), jmax) * kv_dim + vl;
-      vd[0][s] = vr[0];
-      vd[1][s] = vr[32];
+      for (int e = 0; e < 4; ++e) kd[4 * t + e] = __int_as_float(x[e]);
     }
   };
-  float m = -INFINITY, l = 0.0f;
-  f32x16 o0 = {}, o1 = {};
-  auto step = [&](int kbi, const float (&kd)[32], const float (&vd)[2][16]) {
-    f32x16 st = {};
+  auto load_v = [&](int kbi) {
 #pragma unroll
-    for (int s = 0; s < 32; ++s) st = __builtin_amdgcn_mfma_f32_32x32x2f32(kd[s], qb[s], st, 0, 0, 0);
-    float sv[16], mloc = -INFINITY;
+    for (int s = 0; s < 16; ++s) {
+      const int so = (int)((uint32_t)(32 * kbi + attn_key_of(s, 0)) * row_b);
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+        vd[b][s] = __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(vr, voff + 128 * b, so, 0));
+    }
+  };
+  if (w < nkb) load_k(w);
+  for (int i = threadIdx.x; i < kAttnMfmaVecs * (HD / 4); i += 64 * W) {
+    const int v = i / (HD / 4), d = 4 * (i % (HD / 4));
+    const int gv = g0 + v, rv = gv / grp;
+    const float4 x = rv < rows ? *reinterpret_cast<const float4*>(
+                                     q + ((size_t)rv * heads + kvh * grp + gv % grp) * HD + d)
+                               : make_float4(0.f, 0.f, 0.f, 0.f);
+    *reinterpret_cast<float4*>(&Qs[v][d]) = x;
+  }
+  __syncthreads();
+  const float scale = 1.0f / sqrtf((float)HD);
+  float m = -INFINITY, l = 0.0f;
+  f32x16 o[NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) o[b] = f32x16{};
+  int odd = -1;
+  for (int kbi = w; kbi < nkb; kbi += W) {
+    f32x16 st = attn_scores<0, NT>(kd, &Qs[vl][4 * h]);
+    load_v(kbi);
+    load_k(min(kbi + W, nkb - 1));
+    // a hidden key's probability is 0, and 0 * V leaves a sum alone unless V is infinite or NaN: the
+    // blocks that hide keys from some of the vectors look (two blocks at most, so one per wave), and
+    // such a block is added after the others
+    if (32 * kbi + 31 > lim_first) {
+      float z = 0.0f;
+#pragma unroll
+      for (int s = 0; s < 16; ++s)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) z = __builtin_fmaf(vd[b][s], 0.0f, z);
+      if (__ballot(z != z) != 0) {
+        odd = kbi;
+        continue;
+      }
+    }
+    float mloc = -INFINITY;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       const int j = 32 * kbi + attn_key_of(i, h);
-      sv[i] = j <= limit ? st[i] * scale : -INFINITY;
-      mloc = fmaxf(mloc, sv[i]);
+      st[i] = j <= limit ? st[i] * scale : -INFINITY;
+      mloc = fmaxf(mloc, st[i]);
     }
     const float mn = fmaxf(m, fmaxf(mloc, __shfl_xor(mloc, 32, 64)));
-    float pv[16];
-    if (mn == -INFINITY) {               // nothing visible yet for this vector
+    // nothing visible yet for this vector: every term is exp(-inf - 0) = 0
+    const float mref = mn == -INFINITY ? 0.0f : mn;
+    const float alpha = expf(m - mref);  // m = -inf gives 0
+    float ps = 0.0f;
 #pragma unroll
-      for (int i = 0; i < 16; ++i) pv[i] = 0.0f;
-    } else {
-      const float alpha = expf(m - mn);  // m = -inf gives 0
-      float ps = 0.0f;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        pv[i] = expf(sv[i] - mn);
-        ps += pv[i];
-      }
-      l = __builtin_fmaf(l, alpha, ps);
-      o0 *= alpha;
-      o1 *= alpha;
-      m = mn;
+    for (int i = 0; i < 16; ++i) {
+      st[i] = expf(st[i] - mref);
+      ps += st[i];
     }
+    l = __builtin_fmaf(l, alpha, ps);
+    m = mn;
+    // each block's 32 keys are summed from zero and added to the rescaled earlier ones
 #pragma unroll
-    for (int s = 0; s < 16; ++s) {
-      o0 = __builtin_amdgcn_mfma_f32_32x32x2f32(vd[0][s], pv[s], o0, 0, 0, 0);
-      o1 = __builtin_amdgcn_mfma_f32_32x32x2f32(vd[1][s], pv[s], o1, 0, 0, 0);
+    for (int b = 0; b < NB; ++b) {
+      f32x16 t = {};
+#pragma unroll
+      for (int s = 0; s < 16; ++s) t = __builtin_amdgcn_mfma_f32_32x32x2f32(vd[b][s], st[s], t, 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) o[b][i] = __builtin_fmaf(o[b][i], alpha, t[i]);
+      asm volatile("" : "+v"(o[b]));
     }
-  };
-  // two register sets, alternating by hand (a runtime index into them would go to scratch)
-  float kA[32], vA[2][16], kB[32], vB[2][16];
-  if (w < nkb) load(w, kA, vA);
-  for (int kbi = w; kbi < nkb; kbi += 8) {
-    if (kbi + 4 < nkb) load(kbi + 4, kB, vB);
-    step(kbi, kA, vA);
-    if (kbi + 4 >= nkb) break;
-    if (kbi + 8 < nkb) load(kbi + 8, kA, vA);
-    step(kbi + 4, kB, vB);
   }
-  // wave partials: O^T register i of block nb is dim 32 nb + 8(i/4) + 4h + i%4 of vector vl
+  if (__builtin_expect(odd >= 0, 0)) {   // key by key, what each vector sees
+#pragma unroll 1
+    for (int j = 32 * odd; j <= min(32 * odd + 31, jmax); ++j) {
+      const float* kj = kc + (size_t)kvh * HD + (size_t)j * kv_dim + 4 * h;
+      const float* vj = vc + (size_t)kvh * HD + (size_t)j * kv_dim + 4 * h;
+      float s = 0.0f;
+#pragma unroll 1
+      for (int d = 0; d < HD; d += 8)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s = __builtin_fmaf(kj[d + e], Qs[vl][d + 4 * h + e], s);
+      s = (s + __shfl_xor(s, 32, 64)) * scale;
+      if (j > limit) continue;
+      const float mn = fmaxf(m, s), mref = mn == -INFINITY ? 0.0f : mn;
+      const float alpha = expf(m - mref), p = expf(s - mref);
+      l = __builtin_fmaf(l, alpha, h == 0 ? p : 0.0f);   // the halves of l are added below
+      m = mn;
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[b][i] = __builtin_fmaf(o[b][i], alpha, p * vj[32 * b + attn_key_of(i, 0)]);
+    }
+  }
+  // wave partials: O^T register i of block b is dim 32 b + 8(i/4) + 4h + i%4 of vector vl
   l += __shfl_xor(l, 32, 64);
 #pragma unroll
-  for (int i = 0; i < 16; i += 4) {
-    const int d = attn_key_of(i, h);
-    *reinterpret_cast<float4*>(&Os[w][vl][d]) = make_float4(o0[i], o0[i + 1], o0[i + 2], o0[i + 3]);
-    *reinterpret_cast<float4*>(&Os[w][vl][32 + d]) = make_float4(o1[i], o1[i + 1], o1[i + 2], o1[i + 3]);
-  }
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int i = 0; i < 16; i += 4)
+      *reinterpret_cast<float4*>(&Os[w][vl][32 * b + attn_key_of(i, h)]) =
+          make_float4(o[b][i], o[b][i + 1], o[b][i + 2], o[b][i + 3]);
   if (h == 0) {
     Ms[w][vl] = m;
     Ls[w][vl] = l;
   }
   __syncthreads();
-  // combine: thread t -> vector t / 8, dims 8 (t % 8) .. + 7
-  const int v = threadIdx.x >> 3, d0 = 8 * (threadIdx.x & 7);
+  // combine: thread t -> vector t / 16, every 16th four dims from 4 (t % 16)
+  const int v = threadIdx.x >> 4;
   const int gv = g0 + v, rv = gv / grp;
   if (rv >= rows) return;
   float M = Ms[0][v];
 #pragma unroll
-  for (int k = 1; k < 4; ++k) M = fmaxf(M, Ms[k][v]);
-  if (M == -INFINITY) return;            // unreachable for a valid vector (key 0 is visible)
-  float f[4], tot = 0.0f;
+  for (int k = 1; k < W; ++k) M = fmaxf(M, Ms[k][v]);
+  // (every score -inf: the differences are NaN and so is the row, as exp(x - max) gives it)
+  float f[W], tot = 0.0f;
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    f[k] = Ms[k][v] == -INFINITY ? 0.0f : expf(Ms[k][v] - M);
+  for (int k = 0; k < W; ++k) {
+    f[k] = expf(Ms[k][v] - M);
     tot = __builtin_fmaf(Ls[k][v], f[k], tot);
   }
   const float inv = tot != 0.0f ? 1.0f / tot : 1.0f;
-  float outv[8];
+  float* out = ctx + ((size_t)rv * heads + kvh * grp + gv % grp) * HD;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    float a = 0.0f;
+  for (int d = 4 * (threadIdx.x & 15); d < HD; d += 64) {
+    float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) a = __builtin_fmaf(Os[k][v][d0 + e], f[k], a);
-    outv[e] = a * inv;
+    for (int k = 0; k < W; ++k) {
+      const float4 x = *reinterpret_cast<const float4*>(&Os[k][v][d]);
+      a.x = __builtin_fmaf(x.x, f[k], a.x);
+      a.y = __builtin_fmaf(x.y, f[k], a.y);
+      a.z = __builtin_fmaf(x.z, f[k], a.z);
+      a.w = __builtin_fmaf(x.w, f[k], a.w);
+    }
+    *reinterpret_cast<float4*>(out + d) = make_float4(a.x * inv, a.y * inv, a.z * inv, a.w * inv);
   }
-  float* out = ctx + ((size_t)rv * heads + kvh * grp + gv % grp) * HD + d0;
-  *reinterpret_cast<float4*>(out) = make_float4(outv[0], outv[1], outv[2], outv[3]);
-  *reinterpret_cast<float4*>(out + 4) = make_float4(outv[4], outv[5], outv[6], outv[7]);
 }
 
 // q/k/v projection rows (strided; q|k|v may be one fused projection) plus their biases ->
@@ -954,11 +1023,18 @@ hipError_t launch_kv_append(const float* k, const float* v, int rows, int kv_dim
 }
 hipError_t launch_attention(const float* q, const float* kc, const float* vc, int rows, int heads, int kv_heads,
                             int hd, int max_seq, const int* pos, float* work, float* ctx, hipStream_t s) {
-  if (rows >= 8 && hd == 64) {
+  // from 8 rows the matrix cores: 8 rows at position 900 (14 / 2 heads of 64) take 26 us there, one
+  // workgroup per (head, row) with no workspace 29 us, and the gap widens with the rows (300 rows of 8
+  // heads of 32: 9 against 83 us). Other head sizes (up to 256) do not tile by 32, or do not fit the
+  // registers; a cache of 2 GiB or more does not fit the 32-bit offsets. They keep the kernels below.
+  if (rows >= 8 && hd % 32 == 0 && hd <= 128 && (size_t)max_seq * kv_heads * hd * 4 < (1ull << 31)) {
     const int grp = heads / kv_heads;
-    const dim3 grid((unsigned)(((size_t)rows * grp + kAttnMfmaVecs - 1) / kAttnMfmaVecs), (unsigned)kv_heads);
-    hipLaunchKernelGGL(attention_mfma_kernel, grid, dim3(256), 0, s, q, kc, vc, rows, heads, kv_heads, max_seq, pos,
-                       ctx);
+    const dim3 grid((unsigned)(((size_t)rows * grp + kAttnMfmaVecs - 1) / kAttnMfmaVecs * kv_heads));
+    auto* k = hd == 32   ? attention_mfma_kernel<32>
+              : hd == 64 ? attention_mfma_kernel<64>
+              : hd == 96 ? attention_mfma_kernel<96>
+                         : attention_mfma_kernel<128>;
+    hipLaunchKernelGGL(k, grid, dim3(64 * kAttnMfmaWaves), 0, s, q, kc, vc, rows, heads, kv_heads, max_seq, pos, ctx);
     return hipGetLastError();
   }
   if (work) {
