@@ -94,10 +94,11 @@ int re_qmat_matmul_dev(re_qmat *q, const float *d_x, size_t rows, float *d_y, in
                        void *stream);
 /* re_qmat_matmul_dev that allocates nothing, for callers that cannot allocate device memory
  * (code under HIP graph capture, serving loops, harnesses that forbid hipMalloc). It has no
- * counterpart in the reference. The GEMM's K-split partial tiles go to a static device scratch of
- * 32 MiB per GPU instead of a buffer the matrix grows on first use; the same plan, kernels and
- * results as re_qmat_matmul_dev. A plan whose partials exceed the scratch fails with RE_ERR_SIZE
- * (the planned splits of every shape fit: the planner caps partial tiles at 32 MiB). The scratch
+ * counterpart in the reference. The GEMM's K-split partial tiles and packed operands go to a static
+ * device scratch of 64 MiB per GPU instead of buffers allocated on first use; the same plan, kernels
+ * and results as re_qmat_matmul_dev (operands larger than the scratch are packed and multiplied in
+ * pieces). A plan whose partials exceed the scratch fails with RE_ERR_SIZE (the planned splits of
+ * every shape fit: the planner caps partial tiles at 32 MiB). The scratch
  * is shared by every call on a GPU. Outside stream capture, a call on a different stream than the
  * previous call on that GPU first waits for the previous call's launches (an event set up once per
  * device), so calls from several streams or threads stay ordered. Inside stream capture no

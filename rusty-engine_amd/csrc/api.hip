@@ -123,7 +123,7 @@ int check_matrix(uint32_t type, size_t nbytes, size_t m, size_t n, MatGeom* g) {
 // (one copy per GPU, held until the process ends). Host code never passes `scratch` itself to a
 // kernel: that name is a host-side stand-in; g_scratch_dev[dev] holds the device address that
 // hipGetSymbolAddress returns for the device, taken once per device with that device current.
-constexpr size_t kScratchBytes = 32u << 20;
+constexpr size_t kScratchBytes = 64u << 20;
 static __device__ __align__(256) float scratch[kScratchBytes / sizeof(float)];
 
 struct Staging {
@@ -445,6 +445,237 @@ int gemv_enqueue(re_qmat* q, const float* d_x, float* d_y, hipStream_t s, const 
   return RE_OK;
 }
 
+// ---- GEMM over packed bf16 operands (packed.hip) ---------------------------------------------
+// The packed operands live in a workspace only while the call's launches run: up to kPackedSlots
+// buffers per GPU, shared by every matrix (a buffer per matrix would hold another 2-4 bytes per
+// weight). A buffer belongs to one stream at a time, so the stream orders its uses and a call pays
+// for no event (one recorded per call left the GPU idle for 1-4 us). A stream gives its buffer back
+// when a host-pointer call has synchronized it; the buffer of a stream that no longer exists is
+// freed (hipFree waits for the device) and allocated anew. A call that finds no buffer runs on the
+// tiled GEMM. All are freed with the last matrix. (A new stream may get a destroyed stream's handle;
+// the runtime has finished the old stream's work by then.)
+constexpr size_t kPackedWsBytes = 256u << 20;    // largest workspace; larger operands run in pieces
+constexpr int kPackedSlots = 8, kPackedDevices = 64;
+struct PackedSlot {
+  void* p = nullptr;
+  size_t cap = 0;
+  bool owned = false;                             // by `stream`
+  hipStream_t stream = nullptr;
+};
+std::mutex g_packed_mu;
+PackedSlot g_packed[kPackedDevices][kPackedSlots];
+long g_packed_users = 0;                          // live matrices
+
+void packed_user(int delta) {
+  std::lock_guard<std::mutex> lk(g_packed_mu);
+  g_packed_users += delta;
+  if (g_packed_users > 0) return;
+  for (auto& dev : g_packed)
+    for (PackedSlot& sl : dev) {
+      if (sl.p) (void)hipFree(sl.p);              // waits for the work that uses it
+      sl = PackedSlot{};
+    }
+}
+
+// the stream has been synchronized (or is about to go): its buffer is idle
+void packed_idle(hipStream_t s) {
+  std::lock_guard<std::mutex> lk(g_packed_mu);
+  for (auto& dev : g_packed)
+    for (PackedSlot& sl : dev)
+      if (sl.owned && sl.stream == s) sl.owned = false;
+}
+
+// whether the handle still names a stream
+bool stream_lives(hipStream_t s) {
+  unsigned flags = 0;
+  if (!s || hipStreamGetFlags(s, &flags) == hipSuccess) return true;
+  (void)hipGetLastError();
+  return false;
+}
+
+// A buffer of `bytes` for stream s (g_packed_mu held), or nullptr.
+PackedSlot* packed_slot(PackedSlot* slots, size_t bytes, hipStream_t s) {
+  if (s == hipStreamPerThread) return nullptr;    // one handle, but a stream per thread
+  PackedSlot* pick = nullptr;
+  int score = 0;
+  for (int i = 0; i < kPackedSlots; ++i) {
+    PackedSlot& sl = slots[i];
+    const int sc = sl.owned ? (sl.stream == s ? 4 : 0) : !sl.p ? 2 : sl.cap >= bytes ? 3 : 1;
+    if (sc > score) { score = sc; pick = &sl; }
+  }
+  for (int i = 0; i < kPackedSlots && !pick; ++i) {
+    if (stream_lives(slots[i].stream)) continue;
+    pick = &slots[i];                             // its stream is gone
+    (void)hipFree(pick->p);
+    pick->p = nullptr;
+    pick->cap = 0;
+  }
+  if (!pick) return nullptr;
+  if (pick->cap < bytes) {
+    if (pick->p) (void)hipFree(pick->p);
+    *pick = PackedSlot{};
+    if (hipMalloc(&pick->p, bytes) != hipSuccess) {
+      (void)hipGetLastError();
+      pick->p = nullptr;
+      return nullptr;
+    }
+    pick->cap = bytes;
+  }
+  pick->owned = true;
+  pick->stream = s;
+  return pick;
+}
+
+struct PackedCall {
+  uint32_t type;
+  const void* W;
+  int m, K, KB, rows;
+  bool sp;
+  PackedPlan plan;
+  size_t row_bytes() const { return (size_t)(K + 31) / 32 * 64 * (sp ? 2 : 1); }
+  size_t partial_bytes() const {
+    return plan.splits > 1 ? ((size_t)plan.splits * rows * m * sizeof(float) + 255) / 256 * 256 : 0;
+  }
+  // bytes that hold both operands whole, at most `cap`
+  size_t want(size_t cap) const {
+    const size_t all = partial_bytes() + (pad(m) + pad(rows)) * row_bytes();
+    return std::min(all, cap);
+  }
+  static size_t pad(size_t r) { return (r + kPackedRows - 1) / kPackedRows * kPackedRows; }
+};
+
+// Whether packed operands beat decoding in the GEMM, by shape (measured over K 256 .. 14336, m 128 ..
+// 14336 and 64 .. 2048 rows, back to back, us tiled / packed; Q4_K, Q5_0, Q6_K and F16 agree).
+// Packing decodes each weight and converts each activation once, but writes 2 bytes (f32 mode 4) per
+// element and costs a launch.
+//   Quantized weights, whatever the rows: not where the tiled GEMM runs unsplit as one round of
+//   workgroups over a short K (m x K 4864 x 896, 961 rows, bf16: 22.4 / 26.9; 14336 x 512, 512 rows:
+//   19.8 / 27.9; f32 2048 x 768, 961 rows: 21.1 / 25.3).
+//   bf16 mode: from 384 rows (4864 x 896, 512 rows: 26.5 / 18.8; 896 x 896: 17.2 / 13.7), from 192 if
+//   the product is large and K is not short (4096 x 14336, 192 rows: 106 / 68; 4096 x 4096: 36.0 /
+//   31.6; 896 x 896, 320 rows: 10.1 / 13.9).
+//   f32 mode: from 320 rows (4096 x 4096: 102 / 56), from 192 for matrices up to 5M weights (4864 x
+//   896: 25.3 / 23.5; 4096 x 14336, 256 rows: 131 / 186), from 96 up to 1.6M (896 x 896, 128 rows:
+//   19.7 / 13.1; 4864 x 896, 96 rows: 21.7 / 22.2).
+//   Dense weights (F16, bf16 / f32 mode): from 256 rows and 256 weight rows (896 x 896: 14.3 / 13.5;
+//   128 x 896, 1024 rows: 10.1 / 12.9), from 128 rows for 4M weights and more (4864 x 896: 21.1 /
+//   17.3, 23.6 / 22.8; 2048 x 768, f32: 14.6 / 15.9).
+bool packed_pays(bool dense, size_t m, size_t K, size_t rows, bool sp) {
+  if (dense) return (rows >= 256 && m >= 256) || (rows >= 128 && m * K >= 4000000);
+  const GemmPlan pl = plan_gemm((int)m, (int)rows, (int)K, sp ? kGemmModeSplit : RE_MODE_BF16);
+  if (pl.splits == 1 && K <= 1024 && pl.tile != GemmTile::k128x128) {
+    const size_t bm = pl.tile == GemmTile::k64x64 ? 64 : 128;
+    const size_t bn = pl.tile == GemmTile::k64x64 ? 64 : pl.tile == GemmTile::k128x192 ? 192 : 256;
+    const size_t tiles = ((m + bm - 1) / bm) * ((rows + bn - 1) / bn);
+    // one round: a 64 x 64 tile's stages let two workgroups share a CU
+    if (tiles <= (bm == 64 ? 512u : 256u) && tiles > (bm == 64 ? 256u : 128u)) return false;
+  }
+  if (sp) return rows >= 320 || (rows >= 192 && m * K <= 5000000) || (rows >= 96 && m * K <= 1600000);
+  return rows >= 384 || (rows >= 192 && K >= 1024 && (double)m * K * rows >= 3e9);
+}
+
+// Whether a call runs on packed operands, from its shape, type, mode and alignment alone (so that both
+// GEMM entry points take the same kernels). Rows longer than the no-allocation entry point's scratch
+// can hold stay with the tiled GEMM. REHIP_GEMM_PACKED: 0 never, 2 wherever the kernels can.
+bool packed_call(uint32_t type, const void* W, size_t m, size_t K, size_t KB, const float* d_x, size_t rows, int mode,
+                 PackedCall* c) {
+  const bool sp = mode == RE_MODE_F32;
+  const size_t knob = env_size("REHIP_GEMM_PACKED", 1);
+  if (knob == 0 || rows < 2 || !aligned16(d_x)) return false;
+  if (knob != 2 && !packed_pays(dense_type(type), m, K, rows, sp)) return false;
+  if (env_size("REHIP_GEMM_SP", 1) == 0 || env_size("REHIP_GEMM_TILE", 0)) return false;
+  c->type = type;
+  c->W = W;
+  c->m = (int)m;
+  c->K = (int)K;
+  c->KB = (int)KB;
+  c->rows = (int)rows;
+  c->sp = sp;
+  if (2 * kPackedRows * c->row_bytes() > kScratchBytes / 2) return false;
+  c->plan = plan_packed((int)m, (int)rows, (int)K, sp);
+  return true;
+}
+
+// the same for a dense matrix (n % 8 == 0: whole fragment units)
+bool dense_packed(const re_qmat* q, const float* d_x, size_t rows, int mode, PackedCall* c) {
+  return rows <= 65535u * 4u && dense_mma_rows((int)q->g.n, (int)rows, d_x) &&
+         rows * q->g.n * sizeof(float) < (1ull << 31) &&
+         packed_call(q->g.type, q->d_w, q->g.m, q->g.n, 0, d_x, rows, mode, c);
+}
+
+int packed_enqueue(const PackedCall& c, const float* d_x, float* d_y, void* ws, size_t ws_bytes, hipStream_t s) {
+  const size_t rb = c.row_bytes(), part = c.partial_bytes(), avail = ws_bytes - part;
+  const size_t mp = PackedCall::pad(c.m), np = PackedCall::pad(c.rows);
+  size_t mc = mp, nc = np;                       // rows of each operand packed at a time
+  if ((mp + np) * rb > avail) {
+    nc = std::min(np, std::max<size_t>(kPackedRows, avail / 2 / rb / kPackedRows * kPackedRows));
+    mc = std::min(mp, (avail - nc * rb) / rb / kPackedRows * kPackedRows);
+    if (mc == 0) return fail(RE_ERR_SIZE, "packed GEMM workspace of %zu bytes is too small", ws_bytes);
+  }
+  const int KS = (c.K + 31) / 32 * 2, planes = c.sp ? 2 : 1;
+  float* partial = c.plan.splits > 1 ? (float*)ws : nullptr;
+  uint8_t* wp = (uint8_t*)ws + part;
+  uint8_t* xp = wp + mc * rb;
+  for (size_t n0 = 0; n0 < (size_t)c.rows; n0 += nc) {
+    const size_t rows = std::min(nc, c.rows - n0);
+    for (size_t m0 = 0; m0 < (size_t)c.m; m0 += mc) {
+      const size_t mr = std::min(mc, c.m - m0);
+      PackArgs pa{};
+      pa.W = c.W;
+      pa.w_row0 = (int)m0;
+      pa.w_rows = mc == mp && n0 ? 0 : (int)mr;   // one piece of weights stays for every piece of rows
+      pa.K = c.K;
+      pa.KS = KS;
+      pa.KB = c.KB;
+      pa.x = d_x + n0 * c.K;
+      pa.x_rows = m0 ? 0 : (int)rows;
+      pa.Wp = wp;
+      pa.Xp = xp;
+      pa.w_lo = mc * rb / planes;
+      pa.x_lo = nc * rb / planes;
+      HIP_TRY(launch_pack(c.type, pa, c.sp, s));
+      PackedGemmArgs a{};
+      a.Wp = wp;
+      a.Xp = xp;
+      a.w_bytes = (uint32_t)(mc * rb);
+      a.x_bytes = (uint32_t)(nc * rb);
+      a.w_lo = (uint32_t)pa.w_lo;
+      a.x_lo = (uint32_t)pa.x_lo;
+      a.Y = d_y + n0 * c.m + m0;
+      a.partial = partial ? partial + n0 * c.m + m0 : nullptr;
+      a.split_stride = (size_t)c.rows * c.m;
+      a.m = (int)mr;
+      a.N = (int)rows;
+      a.KS = KS;
+      a.ldy = c.m;
+      a.splits = c.plan.splits;
+      a.steps_per_split = c.plan.steps_per_split;
+      HIP_TRY(launch_packed_gemm(a, c.plan.tile, c.sp, s));
+    }
+  }
+  if (partial) HIP_TRY(launch_gemm_reduce(partial, d_y, (size_t)c.rows * c.m, c.plan.splits, s));
+  return RE_OK;
+}
+
+// The call on packed operands, in a workspace of the GPU's; *ran = false (and nothing enqueued) where
+// it cannot be had: under stream capture (a replayed graph would use the shared buffers outside
+// their ordering), no buffer left, or out of memory.
+int packed_shared(const PackedCall& c, const float* d_x, float* d_y, hipStream_t s, bool* ran) {
+  *ran = false;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  HIP_TRY(hipStreamIsCapturing(s, &cs));
+  if (cs != hipStreamCaptureStatusNone) return RE_OK;
+  int dev = 0;
+  HIP_TRY(hipGetDevice(&dev));
+  if (dev < 0 || dev >= kPackedDevices) return RE_OK;
+  const size_t bytes = c.want(kPackedWsBytes);
+  std::lock_guard<std::mutex> lk(g_packed_mu);
+  PackedSlot* sl = packed_slot(g_packed[dev], bytes, s);
+  if (!sl) return RE_OK;
+  *ran = true;
+  return packed_enqueue(c, d_x, d_y, sl->p, bytes, s);
+}
+
 // fixed_partial: nullptr (the matrix's own partial buffer, grown on first use), or a caller-owned
 // buffer of fixed_cap bytes for the split partials (the no-allocation entry point)
 int gemm_enqueue(re_qmat* q, const float* d_x, size_t rows, float* d_y, int mode, hipStream_t s,
@@ -503,6 +734,13 @@ int gemm_enqueue(re_qmat* q, const float* d_x, size_t rows, float* d_y, int mode
       if (a.splits > 1) HIP_TRY(launch_gemm_reduce(a.partial, d_y, rows * q->g.m, a.splits, s));
       return RE_OK;
     }
+  }
+  PackedCall pc;
+  if (packed_call(q->g.type, q->d_w, q->g.m, q->g.n, q->g.kb, d_x, rows, mode, &pc)) {
+    if (fixed_partial) return packed_enqueue(pc, d_x, d_y, fixed_partial, fixed_cap, s);
+    bool ran = false;
+    const int rc = packed_shared(pc, d_x, d_y, s, &ran);
+    if (rc || ran) return rc;
   }
   // f32 mode on bf16 MFMAs with split operands (REHIP_GEMM_SP=0: the f32 MFMA tiles)
   const int kmode = mode == RE_MODE_F32 && env_size("REHIP_GEMM_SP", 1) != 0 ? kGemmModeSplit : mode;
@@ -614,6 +852,7 @@ int create_dense(uint32_t ggml_type, const uint8_t* bytes, size_t nbytes, size_t
   if (rc) return rc;
   re_qmat* q = new (std::nothrow) re_qmat();
   if (!q) return fail(RE_ERR_ARG, "out of memory");
+  packed_user(1);
   q->dense = true;
   q->g.type = ggml_type;
   q->g.m = m;
@@ -648,6 +887,7 @@ int re_qmat_create_stacked(uint32_t ggml_type, const uint8_t* bytes, size_t nbyt
   if ((rc = do_init())) return rc;
   re_qmat* q = new (std::nothrow) re_qmat();
   if (!q) return fail(RE_ERR_ARG, "out of memory");
+  packed_user(1);
   q->g = g;
   q->count = count;
   q->w_stride = (g.bytes + 255) / 256 * 256;
@@ -677,7 +917,10 @@ int re_qmat_create(uint32_t ggml_type, const uint8_t* bytes, size_t nbytes, size
 
 void re_qmat_destroy(re_qmat* q) {
   if (!q) return;
-  if (q->stream) (void)hipStreamSynchronize(q->stream);
+  if (q->stream) {
+    (void)hipStreamSynchronize(q->stream);
+    packed_idle(q->stream);
+  }
   if (q->d_w) (void)hipFree(q->d_w);
   if (q->d_partial) (void)hipFree(q->d_partial);
   if (q->d_norm) (void)hipFree(q->d_norm);
@@ -688,6 +931,7 @@ void re_qmat_destroy(re_qmat* q) {
   q->hy.release();
   if (q->stream) (void)hipStreamDestroy(q->stream);
   delete q;
+  packed_user(-1);
 }
 
 size_t re_qmat_rows(const re_qmat* q) { return q ? q->g.m : 0; }
@@ -821,6 +1065,12 @@ int re_qmat_matmul_dev(re_qmat* q, const float* d_x, size_t rows, float* d_y, in
     // bf16 MFMAs in f32 mode (REHIP_GEMM_SP=0: f32 MFMAs)
     if (rows > 65535u * 4u) return fail(RE_ERR_SIZE, "rows = %zu too large for dense weights", rows);
     const hipStream_t s = (hipStream_t)stream;
+    PackedCall pc;
+    if (dense_packed(q, d_x, rows, mode, &pc)) {
+      bool ran = false;
+      const int rc = packed_shared(pc, d_x, d_y, s, &ran);
+      if (rc || ran) return rc;
+    }
     int splits = 1;
     if (dense_mma_rows((int)q->g.n, (int)rows, d_x)) {
       // few output tiles: K slices into the matrix's partial buffer, grown on first use (under
@@ -877,8 +1127,14 @@ int re_qmat_matmul_noalloc_dev(re_qmat* q, const float* d_x, size_t rows, float*
   if (!q || (rows && (!d_x || !d_y))) return fail(RE_ERR_ARG, "null pointer");
   if (mode != RE_MODE_BF16 && mode != RE_MODE_F32) return fail(RE_ERR_ARG, "unknown mode %d", mode);
   if (rows == 0) return RE_OK;
-  if (rows == 1 || q->dense) return re_qmat_matmul_dev(q, d_x, rows, d_y, mode, stream);   // no scratch
+  PackedCall pc;
+  const bool packed = q->dense && dense_packed(q, d_x, rows, mode, &pc);
+  if (rows == 1 || (q->dense && !packed)) return re_qmat_matmul_dev(q, d_x, rows, d_y, mode, stream);   // no scratch
   if (rows > (1u << 24)) return fail(RE_ERR_SIZE, "rows = %zu too large", rows);
+  auto enqueue = [&](float* scratch_dev, hipStream_t st) {
+    return packed ? packed_enqueue(pc, d_x, d_y, scratch_dev, kScratchBytes, st)
+                  : gemm_enqueue(q, d_x, rows, d_y, mode, st, scratch_dev, kScratchBytes);
+  };
   float* part = nullptr;
   int dev = 0;
   int rc = scratch_for_current_device(&part, &dev);
@@ -887,12 +1143,12 @@ int re_qmat_matmul_noalloc_dev(re_qmat* q, const float* d_x, size_t rows, float*
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   HIP_TRY(hipStreamIsCapturing(s, &cs));
   // under capture the caller orders the replays of graphs that share the scratch
-  if (cs != hipStreamCaptureStatusNone) return gemm_enqueue(q, d_x, rows, d_y, mode, s, part, kScratchBytes);
+  if (cs != hipStreamCaptureStatusNone) return enqueue(part, s);
   // outside capture, calls on different streams of one GPU are ordered through the device's event
   // (the lock also orders calls from different threads); calls on one stream are ordered by it
   std::lock_guard<std::mutex> lk(g_scratch_mu);
   if (g_scratch_used[dev] && g_scratch_last[dev] != s) HIP_TRY(hipStreamWaitEvent(s, g_scratch_ev[dev], 0));
-  if ((rc = gemm_enqueue(q, d_x, rows, d_y, mode, s, part, kScratchBytes))) return rc;
+  if ((rc = enqueue(part, s))) return rc;
   HIP_TRY(hipEventRecord(g_scratch_ev[dev], s));
   g_scratch_last[dev] = s;
   g_scratch_used[dev] = true;
@@ -922,6 +1178,7 @@ int re_qmat_matmul(re_qmat* q, const float* x, size_t rows, float* y, int mode) 
     if ((rc = re_qmat_matmul_dev(q, (const float*)q->sx.p, rows, (float*)q->sy.p, mode, q->stream))) return rc;
     HIP_TRY(hipMemcpyAsync(y, q->sy.p, yb, hipMemcpyDeviceToHost, q->stream));
     HIP_TRY(hipStreamSynchronize(q->stream));
+    packed_idle(q->stream);
     return RE_OK;
   }
   if ((rc = q->hx.ensure(xb)) || (rc = q->hy.ensure(yb))) return rc;
@@ -932,6 +1189,7 @@ int re_qmat_matmul(re_qmat* q, const float* x, size_t rows, float* y, int mode) 
   if ((rc = re_qmat_matmul_dev(q, (const float*)q->sx.p, rows, dy, mode, q->stream))) return rc;
   if (io == 1) HIP_TRY(hipMemcpyAsync(q->hy.h, q->sy.p, yb, hipMemcpyDeviceToHost, q->stream));
   HIP_TRY(hipStreamSynchronize(q->stream));
+  packed_idle(q->stream);
   std::memcpy(y, q->hy.h, yb);
   return RE_OK;
 }

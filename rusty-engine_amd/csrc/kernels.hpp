@@ -156,6 +156,42 @@ GemmPlan plan_gemm(int m, int n, int K, int mode);
 int gemm_kgroups(GemmTile tile, int mode, long workgroups, int steps);
 hipError_t launch_gemm(uint32_t type, int mode, const GemmArgs& a, int ntasks, GemmTile tile, int kgroups,
                        hipStream_t s);
+// GEMM over packed bf16 operands (packed.hip): one launch packs a range of weight rows and
+// activation rows as MFMA fragments, then the GEMM runs on them. KS: k steps of 16 per row,
+// ceil(K / 32) * 2. An operand of r rows takes packed_bytes(r, KS) per plane (two planes in f32 mode).
+constexpr int kPackedRows = 256;          // packed operands are padded to whole tiles of this many rows
+inline size_t packed_bytes(size_t rows, int KS) {
+  return (rows + kPackedRows - 1) / kPackedRows * kPackedRows * (size_t)KS * 32;
+}
+struct PackArgs {
+  const void* W;           // the whole matrix: tiled slabs, or row-major F32 / F16 / BF16
+  int w_row0, w_rows;      // weight rows to pack (w_row0 a multiple of 64; w_rows 0: none)
+  int K, KS, KB;
+  const float* x;          // activation rows to pack (x_rows 0: none)
+  int x_rows;
+  uint8_t *Wp, *Xp;        // packed planes; the remainders' planes w_lo / x_lo bytes further
+  size_t w_lo, x_lo;
+  int w_groups;            // set by launch_pack
+};
+// sp: f32 mode (hi and lo planes). n % 8 == 0 and 16-byte aligned rows for row-major weights and x.
+hipError_t launch_pack(uint32_t type, PackArgs a, bool sp, hipStream_t s);
+enum class PackedTile { k256x256, k256x128, k192x128, k128x128, k128x64 };   // weight rows x activation rows
+struct PackedPlan {
+  PackedTile tile = PackedTile::k128x128;
+  int splits = 1, steps_per_split = 1;
+};
+PackedPlan plan_packed(int m, int rows, int K, bool sp);
+struct PackedGemmArgs {
+  const uint8_t *Wp, *Xp;
+  uint32_t w_bytes, x_bytes;   // all planes
+  uint32_t w_lo, x_lo;
+  float* Y;                // N x m outputs at row stride ldy
+  float* partial;          // splits > 1: slice i writes partial + i * split_stride (row stride ldy)
+  size_t split_stride;
+  int m, N, KS, ldy;
+  int splits, steps_per_split;   // stages of 32 k per slice
+};
+hipError_t launch_packed_gemm(const PackedGemmArgs& a, PackedTile tile, bool sp, hipStream_t s);
 // Few-row dense GEMM (skinny.hip): Y[N x m] = X[N x K] W^T for N <= 64 rows of f32 X, a 64-row
 // weight tile and a K slice of blocks_per_split whole blocks per workgroup; splits > 1 writes
 // partial[split][N][ldy] for the split-K reduce (launch with launch_gemm_reduce).

@@ -1,0 +1,134 @@
+"""The GEMM over packed bf16 operands (packed.hip, REHIP_GEMM_PACKED=2: at every shape it takes)
+against an f64 product, at the edges of its tiles (64 .. 256), fragments (32 rows x 16 k), stages
+(32 k) and K slices; the operands packed in pieces; its workspaces over streams and under capture.
+
+Bounds per output, relative to sum |w x|: bf16 has 8 significant bits, so a rounding is off by at most
+2^-8 and a bf16-mode product by 2^-7 + 2^-16; in f32 mode a remainder is at most 2^-8 of its value and
+its rounding leaves 2^-16, so a product is off by 2^-16 for either operand and 2^-16 for the dropped
+lo x lo (and 2^-32). The f32 sums add K roundings of 2^-24, whatever the MFMAs' order."""
+import numpy as np
+import pytest
+
+import oracle as O
+import rehip
+from rehip import hip, synth
+
+pytestmark = pytest.mark.gpu
+B = hip.DeviceBuffer
+TYPES = [rehip.Q4_0, rehip.Q5_0, rehip.Q8_0, rehip.Q4_K, rehip.Q5_K, rehip.Q6_K, rehip.F32, rehip.F16, rehip.BF16]
+MODES = [rehip.MODE_BF16, rehip.MODE_F32]
+
+
+def weights(rng, t, m, n):
+    v = rng.standard_normal((m, n)).astype(np.float32)
+    if t == rehip.F32:
+        return v.view(np.uint8).reshape(-1)
+    if t == rehip.F16:
+        return v.astype(np.float16).view(np.uint8).reshape(-1)
+    if t == rehip.BF16:
+        return (v.view(np.uint32) >> 16).astype(np.uint16).view(np.uint8).reshape(-1)
+    return synth.weight_bytes(rng, t, m, n)
+
+
+def product(t, w, m, n, x, rows):
+    deq = O.dequant(t, w).reshape(m, -1)[:, :n].astype(np.float64)
+    xx = x.reshape(rows, n).astype(np.float64)
+    return xx @ deq.T, np.abs(xx) @ np.abs(deq).T
+
+
+def check(got, want, n, mode):
+    exact, absd = want
+    rel = (2.0 ** -7 + 2.0 ** -16 if mode == rehip.MODE_BF16 else 3.01 * 2.0 ** -16) + n * 2.0 ** -24
+    assert np.all(np.abs(got.reshape(exact.shape) - exact) <= rel * absd)
+
+
+def run(q, dx, rows, m, mode, call="matmul_dev", stream=None):
+    dy = B(rows * m * 4)
+    getattr(q, call)(dx, rows, dy, mode, stream=stream)
+    hip.synchronize()
+    return dy.download(np.float32, rows * m)
+
+
+@pytest.mark.parametrize("mode", MODES)
+@pytest.mark.parametrize("t", TYPES)
+@pytest.mark.parametrize("m,n,rows", [(1, 32, 65), (64, 64, 128), (70, 256, 100), (193, 96, 257), (129, 4864, 130),
+                                      (257, 1056, 66), (600, 288, 300)])
+def test_against_f64(t, mode, m, n, rows, monkeypatch):
+    monkeypatch.setenv("REHIP_GEMM_PACKED", "2")
+    rng = np.random.default_rng(1000 + t + m + rows)
+    w, x = weights(rng, t, m, n), synth.activations(rng, rows, n)
+    q = rehip.QMat.from_bytes(t, w, m, n)
+    dx, want = B.from_array(x), product(t, w, m, n, x, rows)
+    got = run(q, dx, rows, m, mode)
+    check(got, want, n, mode)
+    assert np.array_equal(run(q, dx, rows, m, mode), got)
+    assert np.array_equal(run(q, dx, rows, m, mode, "matmul_noalloc_dev"), got)
+    q.close()
+
+
+@pytest.mark.parametrize("mode", MODES)
+@pytest.mark.parametrize("m,n,rows", [(4864, 896, 512), (1024, 512, 2100), (300, 2048, 400)])
+def test_planned_tiles(mode, m, n, rows):
+    """Shapes that the planner gives its larger tiles, in the default dispatch."""
+    rng = np.random.default_rng(m + rows)
+    w, x = weights(rng, rehip.Q5_K, m, n), synth.activations(rng, rows, n)
+    q = rehip.QMat.from_bytes(rehip.Q5_K, w, m, n)
+    check(run(q, B.from_array(x), rows, m, mode), product(rehip.Q5_K, w, m, n, x, rows), n, mode)
+    q.close()
+
+
+@pytest.mark.parametrize("t", [rehip.F16, rehip.F32])
+def test_dense_k_remainders(t, monkeypatch):
+    """Dense rows need whole 8-element units only: K that ends inside a fragment and a stage."""
+    monkeypatch.setenv("REHIP_GEMM_PACKED", "2")
+    for n in (8, 24, 40, 200):
+        rng = np.random.default_rng(n)
+        w, x = weights(rng, t, 100, n), synth.activations(rng, 70, n)
+        q = rehip.QMat.from_bytes(t, w, 100, n)
+        for mode in MODES:
+            check(run(q, B.from_array(x), 70, 100, mode), product(t, w, 100, n, x, 70), n, mode)
+        q.close()
+
+
+def test_operands_in_pieces():
+    """Operands beyond the no-allocation scratch are packed and multiplied in pieces: the same bits."""
+    t, m, n, rows = rehip.Q4_0, 700, 16384, 600
+    rng = np.random.default_rng(5)
+    q = rehip.QMat.from_bytes(t, weights(rng, t, m, n), m, n)
+    dx = B.from_array(synth.activations(rng, rows, n))
+    for mode in MODES:
+        assert np.array_equal(run(q, dx, rows, m, mode), run(q, dx, rows, m, mode, "matmul_noalloc_dev"))
+    q.close()
+
+
+def test_streams_and_capture():
+    """More live streams than workspaces, two matrices in turn and no synchronisation in between; then a
+    captured call (the tiled GEMM) replayed between eager ones."""
+    m, n, rows = 640, 512, 400
+    rng = np.random.default_rng(6)
+    qs, dx, want = [], [], []
+    for t in (rehip.Q6_K, rehip.Q8_0):
+        w, x = weights(rng, t, m, n), synth.activations(rng, rows, n)
+        qs.append(rehip.QMat.from_bytes(t, w, m, n))
+        dx.append(B.from_array(x))
+        want.append(product(t, w, m, n, x, rows))
+    streams = [hip.Stream() for _ in range(10)]
+    ys = [B(rows * m * 4) for _ in range(20)]
+    for i in range(20):
+        qs[i % 2].matmul_dev(dx[i % 2], rows, ys[i], rehip.MODE_F32, stream=streams[i // 2])
+    hip.synchronize()
+    for i in range(20):
+        check(ys[i].download(np.float32, rows * m), want[i % 2], n, rehip.MODE_F32)
+    y = B(rows * m * 4)
+    g = hip.Graph(streams[0], lambda: qs[0].matmul_dev(dx[0], rows, y, rehip.MODE_F32, stream=streams[0]))
+    for _ in range(3):
+        g.launch()
+        qs[1].matmul_dev(dx[1], rows, ys[1], rehip.MODE_F32, stream=streams[1])
+        hip.synchronize()
+        check(y.download(np.float32, rows * m), want[0], n, rehip.MODE_F32)
+        check(ys[1].download(np.float32, rows * m), want[1], n, rehip.MODE_F32)
+    g.destroy()
+    for s in streams:
+        s.destroy()
+    for q in qs:
+        q.close()
