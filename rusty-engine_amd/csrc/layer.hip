@@ -353,7 +353,8 @@ template <int NC, bool QKV, bool TAB = false, bool FULL = false>   // kc / vc ar
 __global__ __launch_bounds__(256) void attention_split_kernel(const float* __restrict__ q, const float* kc,
                                                               const float* vc, int heads, int kv_heads,
                                                               int hd, int max_seq, const int* __restrict__ pos,
-                                                              float* __restrict__ work, DecodeQkv dq) {
+                                                              float* __restrict__ work, DecodeQkv dq,
+                                                              float* __restrict__ ctx) {
   constexpr int U = 8;
   __shared__ float sc[kAttnSplitKeys];
   __shared__ float red[4];
@@ -620,6 +621,17 @@ __global__ __launch_bounds__(256) void attention_split_kernel(const float* __res
     }
   }
   __syncthreads();
+  if (ctx) {
+    // the only split: the combine's arithmetic with M = m and a weight of 1
+    const float f = mx == -INFINITY ? 0.0f : 1.0f;
+    const float tot = __builtin_fmaf(((red[0] + red[1]) + red[2]) + red[3], f, 0.0f);
+    const float inv = tot != 0.0f ? 1.0f / tot : 1.0f;
+    for (int d = threadIdx.x; d < hd; d += 256) {
+      const float o = ((part[d] + part[256 + d]) + part[512 + d]) + part[768 + d];
+      ctx[((size_t)r * heads + h) * hd + d] = __builtin_fmaf(o, f, 0.0f) * inv;
+    }
+    return;
+  }
   if (threadIdx.x == 0) {
     wp[0] = mx;
     wp[1] = ((red[0] + red[1]) + red[2]) + red[3];
@@ -1041,17 +1053,18 @@ hipError_t launch_attention(const float* q, const float* kc, const float* vc, in
     const int nsp = (max_seq + kAttnSplitKeys - 1) / kAttnSplitKeys;
     const dim3 grid((unsigned)heads, (unsigned)rows, (unsigned)nsp);
     const DecodeQkv none{};
+    float* one = nsp == 1 ? ctx : nullptr;   // (see launch_attention_decode)
     if (hd <= 64)
       hipLaunchKernelGGL((attention_split_kernel<1, false>), grid, dim3(256), 0, s, q, kc, vc, heads, kv_heads, hd,
-                         max_seq, pos, work, none);
+                         max_seq, pos, work, none, one);
     else if (hd <= 128)
       hipLaunchKernelGGL((attention_split_kernel<2, false>), grid, dim3(256), 0, s, q, kc, vc, heads, kv_heads, hd,
-                         max_seq, pos, work, none);
+                         max_seq, pos, work, none, one);
     else
       hipLaunchKernelGGL((attention_split_kernel<4, false>), grid, dim3(256), 0, s, q, kc, vc, heads, kv_heads, hd,
-                         max_seq, pos, work, none);
+                         max_seq, pos, work, none, one);
     hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+    if (e != hipSuccess || one) return e;
     hipLaunchKernelGGL(attention_combine_kernel, dim3((unsigned)heads, (unsigned)rows), dim3(64), 0, s, work, heads,
                        hd, nsp, ctx);
     return hipGetLastError();
@@ -1081,37 +1094,41 @@ hipError_t launch_attention_decode(const float* q, const float* k, const float* 
                                    hipStream_t s) {
   const int nsp = (max_seq + kAttnSplitKeys - 1) / kAttnSplitKeys;
   const dim3 grid((unsigned)heads, 1u, (unsigned)nsp);
+  // a cache of one split (max_seq <= kAttnSplitKeys): the split kernel writes the context itself and
+  // the combine launch goes (24 layers of 14 / 2 heads of 64, max_seq 128: 37 prompt rows and 23 decode
+  // steps 17.84 -> 16.45 ms, 58 us per step)
+  float* one = nsp == 1 ? ctx : nullptr;
   const DecodeQkv dq{k, v, bq, bk, bv, base, kc, vc, reinterpret_cast<const float2*>(rope), max_seq};
   auto a16 = [](const void* x) { return ((uintptr_t)x & 15) == 0; };   // null passes
   if (rope && hd % 8 == 0 && a16(rope) && a16(q) && a16(k) && a16(v) && a16(bq) && a16(bk) && a16(bv)) {
     if (hd == 64)
       hipLaunchKernelGGL((attention_split_kernel<1, true, true, true>), grid, dim3(256), 0, s, q, kc, vc, heads,
-                         kv_heads, hd, max_seq, pos, work, dq);
+                         kv_heads, hd, max_seq, pos, work, dq, one);
     else if (hd <= 64)
       hipLaunchKernelGGL((attention_split_kernel<1, true, true>), grid, dim3(256), 0, s, q, kc, vc, heads, kv_heads,
-                         hd, max_seq, pos, work, dq);
+                         hd, max_seq, pos, work, dq, one);
     else if (hd <= 128)
       hipLaunchKernelGGL((attention_split_kernel<2, true, true>), grid, dim3(256), 0, s, q, kc, vc, heads, kv_heads,
-                         hd, max_seq, pos, work, dq);
+                         hd, max_seq, pos, work, dq, one);
     else
       hipLaunchKernelGGL((attention_split_kernel<4, true, true>), grid, dim3(256), 0, s, q, kc, vc, heads, kv_heads,
-                         hd, max_seq, pos, work, dq);
+                         hd, max_seq, pos, work, dq, one);
     hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+    if (e != hipSuccess || one) return e;
     hipLaunchKernelGGL(attention_combine_kernel, dim3((unsigned)heads, 1u), dim3(64), 0, s, work, heads, hd, nsp, ctx);
     return hipGetLastError();
   }
   if (hd <= 64)
     hipLaunchKernelGGL((attention_split_kernel<1, true>), grid, dim3(256), 0, s, q, kc, vc, heads, kv_heads, hd,
-                       max_seq, pos, work, dq);
+                       max_seq, pos, work, dq, one);
   else if (hd <= 128)
     hipLaunchKernelGGL((attention_split_kernel<2, true>), grid, dim3(256), 0, s, q, kc, vc, heads, kv_heads, hd,
-                       max_seq, pos, work, dq);
+                       max_seq, pos, work, dq, one);
   else
     hipLaunchKernelGGL((attention_split_kernel<4, true>), grid, dim3(256), 0, s, q, kc, vc, heads, kv_heads, hd,
-                       max_seq, pos, work, dq);
+                       max_seq, pos, work, dq, one);
   hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
+  if (e != hipSuccess || one) return e;
   hipLaunchKernelGGL(attention_combine_kernel, dim3((unsigned)heads, 1u), dim3(64), 0, s, work, heads, hd, nsp, ctx);
   return hipGetLastError();
 }

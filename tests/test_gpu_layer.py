@@ -112,6 +112,30 @@ def test_attention(rows, pos0, nh, nkv, hd):
         rehip.attention_dev(qd, kd, vd, rows, nh, nkv, hd, max_seq, pd, ctx, work=work, work_bytes=wb - 4)
 
 
+@pytest.mark.parametrize("rows,pos0,max_seq", [(1, 0, 1), (1, 127, 128), (3, 40, 100), (7, 121, 128), (2, 130, 128)])
+@pytest.mark.parametrize("nh,nkv,hd", [(14, 2, 64), (3, 1, 100), (2, 2, 256)])
+def test_attention_single_split_equals_combine(nh, nkv, hd, rows, pos0, max_seq):
+    """A cache of one key split writes the context without the combine: the bits of the same cache
+    under a larger max_seq, whose further splits see nothing."""
+    if pos0 + rows > max_seq and rows > 1:
+        rows = 1                                   # past the cache: every row is visible in both
+    rng = np.random.default_rng(rows + pos0 + hd)
+    kvd = nkv * hd
+    kc = np.zeros((400, kvd), np.float32)
+    vc = np.zeros((400, kvd), np.float32)
+    kc[:max_seq] = rng.standard_normal((max_seq, kvd))
+    vc[:max_seq] = rng.standard_normal((max_seq, kvd))
+    qd = B.from_array((2 * rng.standard_normal((rows, nh * hd))).astype(np.float32))
+    out = []
+    for ms, p in ((max_seq, pos0), (400, min(pos0, max_seq - rows))):
+        wb = rehip.attention_work_bytes(rows, nh, hd, ms)
+        ctx = B(rows * nh * hd * 4)
+        rehip.attention_dev(qd, B.from_array(kc), B.from_array(vc), rows, nh, nkv, hd, ms, dev_i32([p]), ctx,
+                            work=B.from_array(np.full(wb // 4, np.nan, np.float32)), work_bytes=wb)
+        out.append(down(ctx, rows * nh * hd))
+    assert np.array_equal(out[0], out[1])
+
+
 def test_attention_split_skips_unwritten_cache_rows():
     """Cache rows past the visible position hold NaN: neither attention path may read them."""
     g = qwen.Geometry(d_model=14 * 64, n_heads=14, n_kv_heads=2)
