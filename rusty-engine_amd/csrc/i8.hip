@@ -60,52 +60,79 @@ __global__ __launch_bounds__(256) void quantize_q8_act_kernel(const float* __res
 constexpr int kI8Chunk = 256;  // blocks of activation scales staged in LDS at a time (n <= 8192: one)
 constexpr int kI8Ahead = 4;    // blocks whose operands are in flight ahead of the MFMA
 
-// Y (rows x m) = Q8_0 W (m x n, tiled slabs) times quantized activations. Workgroup = 2 waves =
-// one 64-row weight tile x 32 activation rows; wave w owns weight rows 32w..32w+31 of the tile.
-// Per block one v_mfma_i32_32x32x32_i8 (A = 32 activation rows x 32 i8, B = 32 i8 x 32 weight
-// rows; lane l supplies row/column l%32 and bytes 16(l/32)..+15 of the block to both, so the
-// i32 sums are the exact block dot products) and the f32 fold of the 16 results the lane holds:
-// activation rows 8(i/4) + 4(l/32) + i%4 of weight row l%32. The activation scales of up to 256
-// blocks are staged in LDS (block-major) once; blocks then go in groups of kI8Ahead with no
-// branch inside a group, the operands of the next group loading while this one is folded (a
-// branch between an MFMA and the reads of its result, or between a load and its use, makes the
-// compiler wait for every outstanding load, or miscount the MFMA's result latency).
-__global__ __launch_bounds__(128) void q8_i8_gemm_kernel(const uint8_t* __restrict__ W, const float* __restrict__ xs,
+// 1.5 * 2^23: an MFMA that starts from these bits leaves the bits of the float kI8Magic + isum
+// (|isum| <= 32 * 128 * 127 < 2^22), so with bias = -kI8Magic * dw (exact: 13 significant bits) one
+// fma gives round(isum * dw), the conversion and the first multiply of the fold in one operation.
+constexpr float kI8Magic = 12582912.0f;
+constexpr int kI8MagicBits = 0x4B400000;
+
+// Y (rows x m) = Q8_0 W (m x n, tiled slabs) times quantized activations. Workgroup = 4 waves = two
+// 64-row weight tiles x 32 activation rows; wave w owns 32 weight rows. Per block one
+// v_mfma_i32_32x32x32_i8 (A = 32 activation rows x 32 i8, B = 32 i8 x 32 weight rows; lane l supplies
+// row/column l%32 and bytes 16(l/32)..+15 of the block to both, so the i32 sums are the exact block dot
+// products) and the f32 fold of the 16 results the lane holds: activation rows 8(i/4) + 4(l/32) + i%4
+// of weight row l%32, three operations each (kI8Magic).
+// The activations go through LDS in stages of kI8Ahead = 4 blocks, one whole 128-byte line of each
+// row (a thread copies one 16-byte unit of a stage, loaded a stage ahead): read per block straight
+// from the rows, an operand load touched 32 lines for 32 bytes of each, and the lines left the L1
+// before their other three blocks were read. The activation scales of up to 256 blocks are staged
+// block-major; weights load into registers kI8Ahead blocks ahead, at a scalar offset. No branch
+// inside a stage (a branch between an MFMA and the reads of its result, or between a load and its
+// use, makes the compiler wait for every outstanding load).
+// 4864 x 896, 961 rows, with the quantization: 34.8 -> 29.2 us (the three-operation fold alone 34.5).
+// A scale that is not finite has no exact bias and leaves NaN: such rows are folded again at the end.
+__global__ __launch_bounds__(256, 4) void q8_i8_gemm_kernel(const uint8_t* __restrict__ W, const float* __restrict__ xs,
                                                          const int8_t* __restrict__ xq, float* __restrict__ y, int m,
-                                                         int n, int rows) {
+                                                         int n, int rows, int tiles) {
 #pragma clang fp contract(off)
   extern __shared__ __align__(16) float dxs_flat[];     // min(nb, kI8Chunk) x 32
   float (*dxs)[32] = reinterpret_cast<float (*)[32]>(dxs_flat);
+  __shared__ uint4 xb[2][32 * 8];                       // 16-byte unit u of row r at r * 8 + (u ^ (r / 2 % 8))
+  constexpr uint32_t SLAB = 64 * 34;
+  static_assert(kI8Ahead == 4, "a stage is one 128-byte line of a row");
   const int nb = n >> 5;
-  const int tile = blockIdx.x, r0 = blockIdx.y * 32;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r0 = blockIdx.y * 32;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tile = min(2 * (int)blockIdx.x + (wave >> 1), tiles - 1);   // past the last: computed, not stored
   const int h = lane >> 5, c = lane & 31;
-  const int trow = wave * 32 + c;                       // weight row inside the tile
-  const uint8_t* wb = W + (size_t)tile * nb * (64 * 34) + h * (64 * 16) + trow * 16;
-  const uint8_t* wd = W + (size_t)tile * nb * (64 * 34) + 2 * (64 * 16) + trow * 2;
-  const int8_t* arow = xq + (size_t)min(r0 + c, rows - 1) * n + 16 * h;
-  v4i A[kI8Ahead], Bw[kI8Ahead];
+  const int trow = (wave & 1) * 32 + c;                 // weight row inside the tile
+  // the tile's slabs and the group's activation rows, each below 2 GiB (n <= 2^24)
+  const __amdgpu_buffer_rsrc_t wr = make_rsrc(W + (size_t)tile * nb * SLAB, (uint32_t)nb * SLAB);
+  const __amdgpu_buffer_rsrc_t ar = make_rsrc(xq + (size_t)r0 * n, (uint32_t)min(32, rows - r0) * (uint32_t)n);
+  const int wo = h * (64 * 16) + trow * 16, wdo = 2 * (64 * 16) + trow * 2;
+  // this thread's unit of a stage (units past the row's end hold the next row's bytes, rows past the
+  // last zeros: neither is used)
+  const int xr = threadIdx.x >> 3, xu = threadIdx.x & 7;
+  const int xo = xr * n + 16 * xu, xd = xr * 8 + (xu ^ ((xr >> 1) & 7));
+  const int nst = (nb + kI8Ahead - 1) / kI8Ahead;
+  auto load_x = [&](int st) __attribute__((always_inline)) {
+    return bld16(ar, (uint32_t)(xo + 128 * min(st, nst - 1)));
+  };
+  v4i Bw[kI8Ahead];
   uint32_t D[kI8Ahead];
+  auto load = [&](const int j, const int kb) __attribute__((always_inline)) {
+    const int kn = min(kb, nb - 1);
+    Bw[j] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wr, wo, kn * (int)SLAB, 0));
+    D[j] = __builtin_amdgcn_raw_buffer_load_b16(wr, wdo, kn * (int)SLAB, 0);
+  };
+  uint4 xv = load_x(0);
 #pragma unroll
-  for (int j = 0; j < kI8Ahead; ++j) {
-    const int kn = min(j, nb - 1);
-    A[j] = *reinterpret_cast<const v4i*>(arow + (size_t)kn * 32);
-    Bw[j] = *reinterpret_cast<const v4i*>(wb + (size_t)kn * (64 * 34));
-    D[j] = *reinterpret_cast<const uint16_t*>(wd + (size_t)kn * (64 * 34));
-  }
+  for (int j = 0; j < kI8Ahead; ++j) load(j, j);
   float s[16];
 #pragma unroll
   for (int i = 0; i < 16; ++i) s[i] = 0.0f;
+  v16i magic;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) magic[i] = kI8MagicBits;
 
   // one block: MFMA on slot j, refill slot j with block kb + kI8Ahead (clamped), fold
-  auto step = [&](const int j, const int kb, const float* dxrow) __attribute__((always_inline)) {
-    const v16i z = {};
-    const v16i acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[j], Bw[j], z, 0, 0, 0);
+  auto step = [&](const int j, const int kb, const uint4* xrow, const float* dxrow) __attribute__((always_inline)) {
+    const v4i a = *reinterpret_cast<const v4i*>(xrow + ((2 * j + h) ^ ((c >> 1) & 7)));
+    const v16i acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, Bw[j], magic, 0, 0, 0);
     const float dw = f16_bits_to_f32(D[j]);
-    const int kn = min(kb + kI8Ahead, nb - 1);
-    A[j] = *reinterpret_cast<const v4i*>(arow + (size_t)kn * 32);
-    Bw[j] = *reinterpret_cast<const v4i*>(wb + (size_t)kn * (64 * 34));
-    D[j] = *reinterpret_cast<const uint16_t*>(wd + (size_t)kn * (64 * 34));
+    const float bias = -kI8Magic * dw;
+    __builtin_amdgcn_sched_barrier(0);    // slot j is free: the refill takes its registers
+    load(j, kb + kI8Ahead);
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       const float4 dx = *reinterpret_cast<const float4*>(dxrow + 8 * g + 4 * h);
@@ -113,48 +140,76 @@ __global__ __launch_bounds__(128) void q8_i8_gemm_kernel(const uint8_t* __restri
 #pragma unroll
       for (int jj = 0; jj < 4; ++jj) {
         const int i = 4 * g + jj;
-        const float t = ((float)acc[i] * dw) * dxv[jj];   // no contraction: fp contract(off) above
+        const float t = __builtin_fmaf(__int_as_float(acc[i]), dw, bias) * dxv[jj];   // not contracted (see above)
         s[i] = s[i] + t;
       }
     }
+    __builtin_amdgcn_sched_barrier(0);   // else every refill moves ahead of the stage's first wait
   };
 
+  const int st = threadIdx.x & 31, sk = threadIdx.x >> 5;   // staging of scales: row, first block
+  const float* srow = xs + (size_t)min(r0 + st, rows - 1) * nb;
+  xb[0][xd] = xv;
+  xv = load_x(1);
+  int buf = 0;
   for (int kb0 = 0; kb0 < nb; kb0 += kI8Chunk) {
     const int kc = min(kI8Chunk, nb - kb0);
-    __syncthreads();
-    // scales of 32 activation rows x kc blocks -> dxs[block][row]; loads issued 8 at a time
-    for (int e0 = threadIdx.x; e0 < kc * 32; e0 += 128 * 8) {
-      float v[8];
+    if (kb0) __syncthreads();
+    // scales of 32 activation rows x kc blocks -> dxs[block][row]; loads issued 4 at a time
+    for (int k0 = sk; k0 < kc; k0 += 8 * 4) {
+      float v[4];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int e = e0 + 128 * u;
-        const int t = e / kc, k = e - t * kc;
-        v[u] = e < kc * 32 ? xs[(size_t)min(r0 + t, rows - 1) * nb + kb0 + k] : 0.0f;
-      }
+      for (int u = 0; u < 4; ++u) v[u] = srow[kb0 + min(k0 + 8 * u, kc - 1)];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int e = e0 + 128 * u;
-        const int t = e / kc, k = e - t * kc;
-        if (e < kc * 32) dxs[k][t] = v[u];
-      }
+      for (int u = 0; u < 4; ++u)
+        if (k0 + 8 * u < kc) dxs[k0 + 8 * u][st] = v[u];
     }
-    __syncthreads();
     const int full = kc & ~(kI8Ahead - 1);
+#pragma unroll 1
     for (int k = 0; k < full; k += kI8Ahead) {
+      __syncthreads();                    // the stage is there; everyone has read the one before it
+      xb[buf ^ 1][xd] = xv;
+      xv = load_x((kb0 + k) / kI8Ahead + 2);
+      __builtin_amdgcn_sched_barrier(0);
+      const uint4* xrow = xb[buf] + c * 8;
 #pragma unroll
-      for (int j = 0; j < kI8Ahead; ++j) step(j, kb0 + k + j, dxs[k + j]);
+      for (int j = 0; j < kI8Ahead; ++j) step(j, kb0 + k + j, xrow, dxs[k + j]);
+      buf ^= 1;
     }
-    // blocks past the last whole group (only in the last chunk: kI8Chunk is a multiple of 4)
-#pragma unroll
-    for (int j = 0; j < kI8Ahead - 1; ++j)
-      if (full + j < kc) step(j, kb0 + full + j, dxs[full + j]);
   }
-  const int wr = tile * 64 + trow;
-  if (wr >= m) return;
+  // blocks past the last whole stage (only in the last chunk: kI8Chunk is a multiple of 4)
+  __syncthreads();
+  const int tail = nb & ~(kI8Ahead - 1);
+#pragma unroll
+  for (int j = 0; j < kI8Ahead - 1; ++j)
+    if (tail + j < nb) step(j, tail + j, xb[buf] + c * 8, dxs[(tail & (kI8Chunk - 1)) + j]);
+  bool nan = false;                       // inf * dw - inf: every sum of such a row is NaN
+#pragma unroll
+  for (int i = 0; i < 16; ++i) nan |= s[i] != s[i];
+  if (__any(nan)) {
+    const int8_t* arow = xq + (size_t)min(r0 + c, rows - 1) * n + 16 * h;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s[i] = 0.0f;
+#pragma unroll 1
+    for (int kb = 0; kb < nb; ++kb) {
+      load(0, kb);
+      const v4i a = *reinterpret_cast<const v4i*>(arow + (size_t)kb * 32);
+      const v16i acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, Bw[0], v16i{}, 0, 0, 0);
+      const float dw = f16_bits_to_f32(D[0]);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const float dx = xs[(size_t)min(r0 + 8 * (i >> 2) + 4 * h + (i & 3), rows - 1) * nb + kb];
+        const float t = ((float)acc[i] * dw) * dx;
+        s[i] = s[i] + t;
+      }
+    }
+  }
+  const int wrow = tile * 64 + trow;
+  if (wrow >= m || 2 * (int)blockIdx.x + (wave >> 1) >= tiles) return;
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
     const int r = r0 + 8 * (i >> 2) + 4 * h + (i & 3);
-    if (r < rows) y[(size_t)r * m + wr] = s[i];
+    if (r < rows) y[(size_t)r * m + wrow] = s[i];
   }
 }
 
@@ -339,15 +394,17 @@ hipError_t launch_q8_i8_gemm(const uint8_t* W, int tiles, const float* xs, const
     return hipGetLastError();
   }
   const unsigned rgroups = (unsigned)((rows + 31) / 32);
-  // long rows over few output tiles: split each tile's fold over the waves of a workgroup
-  if ((n >> 5) >= 64 && (size_t)tiles * 2 * rgroups < 512) {
+  // long rows over few output tiles: split each tile's fold over the waves of a workgroup (and rows past
+  // the 32-bit offsets of the other kernel)
+  if ((n >> 5) >= 64 && ((size_t)tiles * 2 * rgroups < 512 || n > (1 << 24))) {
     const size_t lds = (size_t)min(n >> 5, kI8Chunk) * 32 * sizeof(float);
     hipLaunchKernelGGL(q8_i8_gemm_seg_kernel, dim3((unsigned)tiles * 2, rgroups), dim3(64 * kSegWaves), lds, s, W,
                        xs, xq, y, m, n, rows);
     return hipGetLastError();
   }
   const size_t lds = (size_t)min(n >> 5, kI8Chunk) * 32 * sizeof(float);
-  hipLaunchKernelGGL(q8_i8_gemm_kernel, dim3((unsigned)tiles, rgroups), dim3(128), lds, s, W, xs, xq, y, m, n, rows);
+  hipLaunchKernelGGL(q8_i8_gemm_kernel, dim3((unsigned)(tiles + 1) / 2, rgroups), dim3(256), lds, s, W, xs, xq, y, m, n,
+                     rows, tiles);
   return hipGetLastError();
 }
 

@@ -110,6 +110,36 @@ def test_matmul_i8_full_size_sampled_rows(m, n):
     q.close()
 
 
+@pytest.mark.parametrize("m,n,rows", [(70, 96, 33), (1030, 8224, 35), (64, 160, 65)])
+def test_matmul_i8_extreme_scales(m, n, rows):
+    """Rows whose scales are infinite, NaN, zero, subnormal or the largest finite, beside ordinary ones,
+    with quants of -128 (the fold's one-fma product is exact only for finite scales)."""
+    rng = np.random.default_rng(m + n)
+    w = synth.weight_bytes(rng, rehip.Q8_0, m, n).reshape(m, n // 32, 34).copy()
+    d = w[:, :, :2].copy().view(np.float16)[..., 0]
+    for row, v in ((0, np.inf), (3, -np.inf), (5, np.nan), (7, 0.0), (9, -0.0), (11, 6e-8), (13, 65504.0)):
+        d[row, row % (n // 32)] = v
+    d[63] = np.float16(np.inf)
+    w[:, :, :2] = d[..., None].view(np.uint8).reshape(m, n // 32, 2)
+    w[33, :, 2:] = 0x80
+    w[34, :, 2:] = 0
+    w = w.reshape(-1)
+    x = activations(rng, rows, n)
+    sc, qs = oracle_rows(x, rows, n)
+    q = rehip.QMat.from_bytes(rehip.Q8_0, w, m, n)
+    got = q.matmul_i8(sc, qs, rows).reshape(rows, m)
+    with np.errstate(invalid="ignore", over="ignore"):
+        # the fold of the definition: s += ((f32)isum * dw) * dx, block by block
+        want = np.zeros((rows, m), np.float32)
+        wq = w.reshape(m, n // 32, 34)[:, :, 2:].copy().view(np.int8).astype(np.int64)
+        xq, scr = qs.reshape(rows, n // 32, 32).astype(np.int64), sc.reshape(rows, -1)
+        for kb in range(n // 32):
+            isum = (xq[:, kb] @ wq[:, kb].T).astype(np.float32)
+            want += (isum * d[None, :, kb].astype(np.float32)) * scr[:, kb, None]
+    assert np.array_equal(got, want, equal_nan=True)
+    q.close()
+
+
 def test_errors():
     rng = np.random.default_rng(1)
     q = rehip.QMat.from_bytes(rehip.Q4_K, synth.weight_bytes(rng, rehip.Q4_K, 64, 256), 64, 256)
