@@ -288,6 +288,14 @@ int re_ffn_create(re_qmat *gate, re_qmat *up, re_ffn **out);
 void re_ffn_destroy(re_ffn *f);
 /* d_norm_w: NULL, or x is RMS-normalised first (the FFN norm, forward.rs:479). */
 int re_ffn_forward_dev(re_ffn *f, const float *d_x, const float *d_norm_w, float eps, float *d_h, void *stream);
+/* A whole FFN over several rows (prefill): y = add + down(silu(gate x) * up x), x `rows` rows of gate's
+ * columns (already normalised), add NULL or `rows` rows of down's rows (may be y: the residual). The
+ * results of the two products, SwiGLU, the down product and the addition as calls of their own; from a
+ * few hundred rows of quantized weights the products and SwiGLU are one GEMM. d_work: at least
+ * re_ffn_block_work_bytes(f, down, rows) bytes of device memory. */
+size_t re_ffn_block_work_bytes(const re_ffn *f, const re_qmat *down, size_t rows);
+int re_ffn_block_dev(re_ffn *f, re_qmat *down, const float *d_x, size_t rows, const float *d_add, float *d_y,
+                     float *d_work, size_t work_bytes, int mode, void *stream);
 
 /* ---- int8 activations (src/kernel.rs:70-166) ------------------------------------------
  * re_quantize_q8_act[_dev]: Q8Activation::from_f32 (kernel.rs:88-105) of `rows` activation rows

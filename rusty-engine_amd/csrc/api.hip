@@ -454,7 +454,7 @@ int gemv_enqueue(re_qmat* q, const float* d_x, float* d_y, hipStream_t s, const 
 // freed (hipFree waits for the device) and allocated anew. A call that finds no buffer runs on the
 // tiled GEMM. All are freed with the last matrix. (A new stream may get a destroyed stream's handle;
 // the runtime has finished the old stream's work by then.)
-constexpr size_t kPackedWsBytes = 256u << 20;    // largest workspace; larger operands run in pieces
+constexpr size_t kPackedWsBytes = 512u << 20;    // largest workspace; larger operands run in pieces
 constexpr int kPackedSlots = 8, kPackedDevices = 64;
 struct PackedSlot {
   void* p = nullptr;
@@ -674,6 +674,132 @@ int packed_shared(const PackedCall& c, const float* d_x, float* d_y, hipStream_t
   if (!sl) return RE_OK;
   *ran = true;
   return packed_enqueue(c, d_x, d_y, sl->p, bytes, s);
+}
+
+// Whether a whole FFN on packed operands beats its separate calls (each by its own best route), by shape
+// (d x ff 896 x 4864, 1024 x 2816, 2048 x 5632, 2048 x 8192, 3584 x 9472 and 4096 x 14336, 64 .. 2048 rows,
+// back to back, us separate / block). Up to 17M weights a matrix from 128 rows in bf16 mode (896 x 4864:
+// 64 rows 37.0 / 38.5, 128 rows 40.2 / 38.9, 256 rows 66.7 / 38.7, 961 rows 89.8 / 57.2; 2048 x 8192: 64 rows
+// 48.0 / 57.4, 128 rows 63.1 / 56.4) and from 64 in f32 mode (1024 x 2816: 46.3 / 42.5; 896 x 4864, 961 rows:
+// 133.9 / 104.9). Larger matrices take longer to write packed than a few hundred rows gain (4096 x 14336,
+// 384 rows: 245 / 264; f32 mode, 128 rows: 222 / 341): from 768 rows (961 rows: 477 / 436, 1036 / 947).
+bool packed_ffn_pays(size_t ff, size_t K, size_t rows, bool sp) {
+  if (ff * K > 17000000) return rows >= 768;
+  return rows >= (sp ? 64u : 128u);
+}
+
+// y = (add +) down(silu(gate x) * up x) on packed operands: gate and up packed as alternating 32-row
+// groups and multiplied by one GEMM whose epilogue writes h as the down projection's packed
+// activations (the rounding that packing the f32 h would give), so neither gate, up nor h are ever
+// in memory in f32 and x is packed once; the residual is added in the down GEMM's epilogue or reduce.
+// Weights larger than the workspace go in pieces. 961-row prefill of 24 layers (896 x 4864): 4271 -> 3629 us.
+// *ran = false (and nothing enqueued) where the rule or the workspace says no.
+int packed_ffn(const re_qmat* gate, const re_qmat* up, const re_qmat* down, const float* d_x, size_t rows,
+               const float* d_add, float* d_y, int mode, hipStream_t s, bool* ran) {
+  *ran = false;
+  const size_t ff = gate->g.m, d = down->g.m;
+  if (gate->dense || down->dense || gate->count != 1 || up->count != 1 || down->count != 1 || ff % 32) return RE_OK;
+  const bool sp = mode == RE_MODE_F32;
+  const size_t knob = env_size("REHIP_GEMM_PACKED", 1);
+  if (knob == 0 || rows < 2 || rows >= (1u << 20) || 2 * ff >= (1u << 24) || !aligned16(d_x)) return RE_OK;
+  if (env_size("REHIP_GEMM_SP", 1) == 0 || env_size("REHIP_GEMM_TILE", 0)) return RE_OK;
+  if (knob != 2 && !packed_ffn_pays(ff, gate->g.n, rows, sp)) return RE_OK;
+  PackedCall c1{gate->g.type, gate->d_w, (int)(2 * ff), (int)gate->g.n, (int)gate->g.kb, (int)rows, sp, {}};
+  PackedCall c2{down->g.type, down->d_w, (int)d, (int)ff, (int)down->g.kb, (int)rows, sp, {}};
+  c1.plan = plan_packed(c1.m, c1.rows, c1.K, sp, true);
+  c2.plan = plan_packed(c2.m, c2.rows, c2.K, sp);
+  // the K-slice partials, x, h, and a region for packed weights: pieces of gate and up, then of down
+  const size_t rb1 = c1.row_bytes(), rb2 = c2.row_bytes(), part = c2.partial_bytes();
+  const size_t xb = PackedCall::pad(rows) * rb1, hb = PackedCall::pad(rows) * rb2, fixed = part + xb + hb;
+  if (fixed + kPackedWsBytes / 8 > kPackedWsBytes) return RE_OK;
+  const size_t region = std::min(std::max(PackedCall::pad(2 * ff) * rb1, PackedCall::pad(d) * rb2), kPackedWsBytes - fixed);
+  // pieces of equal size, in whole tiles
+  auto piece = [&](size_t all, size_t rb) {
+    const size_t most = region / rb / kPackedRows * kPackedRows;
+    return most ? PackedCall::pad((all + (all + most - 1) / most - 1) / ((all + most - 1) / most)) : 0;
+  };
+  const size_t fc = piece(2 * ff, rb1) / 2, dc = piece(d, rb2);   // fc rows of gate and fc of up
+  if (fc == 0 || dc == 0) return RE_OK;
+  const size_t total = fixed + region;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  HIP_TRY(hipStreamIsCapturing(s, &cs));
+  if (cs != hipStreamCaptureStatusNone) return RE_OK;
+  int dev = 0;
+  HIP_TRY(hipGetDevice(&dev));
+  if (dev < 0 || dev >= kPackedDevices) return RE_OK;
+  std::lock_guard<std::mutex> lk(g_packed_mu);
+  PackedSlot* sl = packed_slot(g_packed[dev], total, s);
+  if (!sl) return RE_OK;
+  *ran = true;
+  uint8_t* ws = (uint8_t*)sl->p;
+  uint8_t *xp = ws + part, *hp = xp + xb, *wp = hp + hb;
+  const int planes = sp ? 2 : 1, KS1 = (c1.K + 31) / 32 * 2, KS2 = (c2.K + 31) / 32 * 2;
+  for (size_t f0 = 0; f0 < ff; f0 += fc) {      // fc is a multiple of 128: whole slabs and h fragments
+    PackArgs pa{};
+    pa.W = gate->d_w;
+    pa.W2 = up->d_w;
+    pa.w_row0 = (int)f0;
+    pa.w_rows = (int)std::min(fc, ff - f0);
+    pa.K = c1.K;
+    pa.KS = KS1;
+    pa.KB = c1.KB;
+    pa.x = d_x;
+    pa.x_rows = f0 ? 0 : (int)rows;
+    pa.Wp = wp;
+    pa.Xp = xp;
+    pa.w_lo = 2 * fc * rb1 / planes;
+    pa.x_lo = xb / planes;
+    HIP_TRY(launch_pack(c1.type, pa, sp, s));
+    PackedGemmArgs a{};
+    a.Wp = wp;
+    a.Xp = xp;
+    a.w_bytes = (uint32_t)(2 * fc * rb1);
+    a.x_bytes = (uint32_t)xb;
+    a.w_lo = (uint32_t)pa.w_lo;
+    a.x_lo = (uint32_t)pa.x_lo;
+    a.m = 2 * pa.w_rows;
+    a.N = (int)rows;
+    a.KS = KS1;
+    a.splits = 1;
+    a.steps_per_split = c1.plan.steps_per_split;
+    a.Hp = hp + f0 / 16 * 1024;
+    a.h_lo = (uint32_t)(hb / planes);
+    a.KSh = KS2;
+    HIP_TRY(launch_packed_gemm(a, c1.plan.tile, sp, s));
+  }
+  float* partial = c2.plan.splits > 1 ? (float*)ws : nullptr;
+  for (size_t m0 = 0; m0 < d; m0 += dc) {
+    PackArgs pd{};
+    pd.W = down->d_w;
+    pd.w_row0 = (int)m0;
+    pd.w_rows = (int)std::min(dc, d - m0);
+    pd.K = c2.K;
+    pd.KS = KS2;
+    pd.KB = c2.KB;
+    pd.Wp = wp;
+    pd.w_lo = dc * rb2 / planes;
+    HIP_TRY(launch_pack(c2.type, pd, sp, s));
+    PackedGemmArgs b{};
+    b.Wp = wp;
+    b.Xp = hp;
+    b.w_bytes = (uint32_t)(dc * rb2);
+    b.x_bytes = (uint32_t)hb;
+    b.w_lo = (uint32_t)pd.w_lo;
+    b.x_lo = (uint32_t)(hb / planes);
+    b.Y = d_y + m0;
+    b.partial = partial ? partial + m0 : nullptr;
+    b.split_stride = rows * d;
+    b.m = pd.w_rows;
+    b.N = (int)rows;
+    b.KS = KS2;
+    b.ldy = c2.m;
+    b.splits = c2.plan.splits;
+    b.steps_per_split = c2.plan.steps_per_split;
+    b.add = partial || !d_add ? nullptr : d_add + m0;   // else in the reduce
+    HIP_TRY(launch_packed_gemm(b, c2.plan.tile, sp, s));
+  }
+  if (partial) HIP_TRY(launch_gemm_reduce(partial, d_y, rows * d, c2.plan.splits, s, d_add));
+  return RE_OK;
 }
 
 // fixed_partial: nullptr (the matrix's own partial buffer, grown on first use), or a caller-owned
@@ -2336,6 +2462,38 @@ int re_ffn_forward_dev(re_ffn* f, const float* d_x, const float* d_norm_w, float
   g.ldy = (int)f->gate->g.m;
   g.max_rows = 1;
   HIP_TRY(launch_moe_gemv(f->gate->g.type, true, g, f->ntasks, (hipStream_t)stream));
+  return RE_OK;
+}
+
+size_t re_ffn_block_work_bytes(const re_ffn* f, const re_qmat* down, size_t rows) {
+  if (!f || !down || rows == 0) return 0;
+  auto pad = [](size_t v) { return (v + 63) / 64 * 64; };
+  return (3 * pad(rows * f->gate->g.m) + pad(rows * down->g.m)) * sizeof(float);
+}
+
+int re_ffn_block_dev(re_ffn* f, re_qmat* down, const float* d_x, size_t rows, const float* d_add, float* d_y,
+                     float* d_work, size_t work_bytes, int mode, void* stream) {
+  if (!f || !down || (rows && (!d_x || !d_y || !d_work))) return fail(RE_ERR_ARG, "null pointer");
+  if (mode != RE_MODE_BF16 && mode != RE_MODE_F32) return fail(RE_ERR_ARG, "unknown mode %d", mode);
+  if (down->g.n != f->gate->g.m)
+    return fail(RE_ERR_SIZE, "ffn block: down takes %zu columns, gate and up give %zu", down->g.n, f->gate->g.m);
+  if (rows == 0) return RE_OK;
+  if (rows > (1u << 24)) return fail(RE_ERR_SIZE, "rows = %zu too large", rows);
+  if (work_bytes < re_ffn_block_work_bytes(f, down, rows))
+    return fail(RE_ERR_SIZE, "ffn block workspace of %zu bytes, need %zu", work_bytes,
+                re_ffn_block_work_bytes(f, down, rows));
+  const hipStream_t s = (hipStream_t)stream;
+  bool ran = false;
+  int rc = packed_ffn(f->gate, f->up, down, d_x, rows, d_add, d_y, mode, s, &ran);
+  if (rc || ran) return rc;
+  auto pad = [](size_t v) { return (v + 63) / 64 * 64; };
+  const size_t nh = rows * f->gate->g.m;
+  float *g = d_work, *u = g + pad(nh), *h = u + pad(nh), *o = d_add ? h + pad(nh) : d_y;
+  if ((rc = re_qmat_matmul_dev(f->gate, d_x, rows, g, mode, stream))) return rc;
+  if ((rc = re_qmat_matmul_dev(f->up, d_x, rows, u, mode, stream))) return rc;
+  HIP_TRY(launch_swiglu(g, u, h, nh, s));
+  if ((rc = re_qmat_matmul_dev(down, h, rows, o, mode, stream))) return rc;
+  if (d_add) HIP_TRY(launch_add(d_add, o, rows * down->g.m, rows * down->g.m, d_y, s));
   return RE_OK;
 }
 

@@ -618,13 +618,16 @@ __device__ __forceinline__ void store_final(float* p, float v) { __builtin_nonte
 __device__ __forceinline__ void store_final(float4* p, float4 v) {
   __builtin_nontemporal_store(f32x4_t{v.x, v.y, v.z, v.w}, reinterpret_cast<f32x4_t*>(p));
 }
-template <typename V>
-__global__ __launch_bounds__(256) void gemm_reduce_kernel(const V* __restrict__ partial, V* __restrict__ y, size_t n,
-                                                          int splits) {
+// ADD: y = add + the sum (add may be y)
+template <typename V, bool ADD>
+__global__ __launch_bounds__(256) void gemm_reduce_kernel(const V* __restrict__ partial, V* y, size_t n, int splits,
+                                                          const V* add) {
   const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= n) return;
   // up to sixteen slices' loads in flight per round trip (the slice count is uniform, so the
   // guards are scalar branches); the sum runs in slice order
+  V a;
+  if constexpr (ADD) a = add[i];
   V s = partial[i];
   for (int sp = 1; sp < splits; sp += 16) {
     V v[16];
@@ -635,23 +638,26 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const V* __restrict__ 
     for (int j = 0; j < 16; ++j)
       if (sp + j < splits) s = vadd(s, v[j]);
   }
+  if constexpr (ADD) s = vadd(a, s);
   store_final(y + i, s);
 }
 
-static hipError_t launch_reduce(const float* partial, float* y, size_t n, int splits, hipStream_t s) {
-  if (n % 4 == 0 && ((uintptr_t)partial & 15) == 0 && ((uintptr_t)y & 15) == 0) {
+static hipError_t launch_reduce(const float* partial, float* y, size_t n, int splits, hipStream_t s,
+                                const float* add = nullptr) {
+  if (n % 4 == 0 && ((uintptr_t)partial & 15) == 0 && ((uintptr_t)y & 15) == 0 && ((uintptr_t)add & 15) == 0) {
     const size_t n4 = n / 4;
-    hipLaunchKernelGGL(gemm_reduce_kernel<float4>, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s,
-                       (const float4*)partial, (float4*)y, n4, splits);
+    auto* k = add ? gemm_reduce_kernel<float4, true> : gemm_reduce_kernel<float4, false>;
+    hipLaunchKernelGGL(k, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s, (const float4*)partial, (float4*)y, n4,
+                       splits, (const float4*)add);
   } else {
-    hipLaunchKernelGGL(gemm_reduce_kernel<float>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, partial, y, n,
-                       splits);
+    auto* k = add ? gemm_reduce_kernel<float, true> : gemm_reduce_kernel<float, false>;
+    hipLaunchKernelGGL(k, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, partial, y, n, splits, add);
   }
   return hipGetLastError();
 }
 
-hipError_t launch_gemm_reduce(const float* partial, float* y, size_t n, int splits, hipStream_t s) {
-  return launch_reduce(partial, y, n, splits, s);
+hipError_t launch_gemm_reduce(const float* partial, float* y, size_t n, int splits, hipStream_t s, const float* add) {
+  return launch_reduce(partial, y, n, splits, s, add);
 }
 
 // x[i] -> bf16 with round to nearest even (the rounding the bf16-mode GEMM applies to f32 X), 8

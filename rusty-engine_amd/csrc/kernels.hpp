@@ -169,6 +169,8 @@ struct PackArgs {
   int K, KS, KB;
   const float* x;          // activation rows to pack (x_rows 0: none)
   int x_rows;
+  const void* W2 = nullptr;   // quantized only: a second matrix of the same shape; groups of 32 rows of W
+                              // and W2 then alternate in Wp (w_row0 0, w_rows a multiple of 32)
   uint8_t *Wp, *Xp;        // packed planes; the remainders' planes w_lo / x_lo bytes further
   size_t w_lo, x_lo;
   int w_groups;            // set by launch_pack
@@ -180,7 +182,8 @@ struct PackedPlan {
   PackedTile tile = PackedTile::k128x128;
   int splits = 1, steps_per_split = 1;
 };
-PackedPlan plan_packed(int m, int rows, int K, bool sp);
+// pairs: the SwiGLU epilogue (one K slice, whole gate / up pairs per wave)
+PackedPlan plan_packed(int m, int rows, int K, bool sp, bool pairs = false);
 struct PackedGemmArgs {
   const uint8_t *Wp, *Xp;
   uint32_t w_bytes, x_bytes;   // all planes
@@ -190,6 +193,12 @@ struct PackedGemmArgs {
   size_t split_stride;
   int m, N, KS, ldy;
   int splits, steps_per_split;   // stages of 32 k per slice
+  const float* add = nullptr;    // splits 1: added to Y (may be Y); row stride ldy
+  // SwiGLU epilogue instead of Y: W holds alternating 32-row groups of gate and up, m counts both;
+  // h = silu(gate) * up goes to Hp as packed activations of m / 2 columns (KSh k steps)
+  uint8_t* Hp = nullptr;
+  uint32_t h_lo = 0;
+  int KSh = 0;
 };
 hipError_t launch_packed_gemm(const PackedGemmArgs& a, PackedTile tile, bool sp, hipStream_t s);
 // Few-row dense GEMM (skinny.hip): Y[N x m] = X[N x K] W^T for N <= 64 rows of f32 X, a 64-row
@@ -215,7 +224,9 @@ size_t skinny_lds_bytes(int staged_k, bool split_operands);
 // split_operands: f32 mode (split bf16 operands, three MFMAs per product)
 hipError_t launch_gemm_skinny(uint32_t type, const SkinnyArgs& a, bool split_operands, hipStream_t s);
 // y = sum over splits, in split order, of partial[split] (n floats each), streaming stores
-hipError_t launch_gemm_reduce(const float* partial, float* y, size_t n, int splits, hipStream_t s);
+// y = (add +) the slices' sum; add may be y
+hipError_t launch_gemm_reduce(const float* partial, float* y, size_t n, int splits, hipStream_t s,
+                              const float* add = nullptr);
 
 // xb[i] = bf16(x[i]), round to nearest even; n a multiple of 8, both buffers 16-byte aligned
 hipError_t launch_x_to_bf16(const float* x, void* xb, size_t n, hipStream_t s);

@@ -29,6 +29,7 @@ namespace rehip {
 namespace {
 
 typedef __attribute__((address_space(3))) void lds_void_t;
+typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4_t;
 
 // s_waitcnt vmcnt(N) lgkmcnt(0): at most N copies of this wave still in flight, every fragment read
 // done (the builtin, so the compiler's own wait counting sees it)
@@ -113,12 +114,16 @@ __device__ __forceinline__ void pack_rows(const void* src, int rows, int K, int 
 // One wave packs one 32-quant chunk of a slab's 64 rows (lane = row): the four units of the
 // chunk's two 16-element runs.
 template <int T, bool SP>
-__device__ __forceinline__ void pack_chunk(const PackArgs& p, int tile, int c) {
+__device__ __forceinline__ void pack_chunk(const PackArgs& p, const void* W, int tile, int c) {
   using B = Blk<T>;
   const int lane = threadIdx.x & 63;
   const int kb = c / B::NCH, cc = c - kb * B::NCH;
-  const uint8_t* slab = (const uint8_t*)p.W + ((size_t)tile * p.KB + kb) * B::SLAB;
-  const int row = 64 * tile + lane - p.w_row0;
+  const uint8_t* slab = (const uint8_t*)W + ((size_t)tile * p.KB + kb) * B::SLAB;
+  int row = 64 * tile + lane - p.w_row0;
+  if (p.W2) {
+    if (row >= p.w_rows) return;          // (the other matrix's groups would follow)
+    row = 2 * row - (row & 31) + (W == p.W2 ? 32 : 0);
+  }
   Run a, b;
   B::chunk(slab, lane, cc, a, b);
 #pragma unroll
@@ -157,9 +162,10 @@ __global__ __launch_bounds__(256) void pack_kernel(PackArgs p) {
                        p.w_lo);
     } else {
       const int nch = p.KB * Blk<(int)T>::NCH;
-      const int t = job / nch;
-      if (t >= (p.w_rows + 63) / 64) return;
-      pack_chunk<(int)T, SP>(p, p.w_row0 / 64 + t, job - t * nch);
+      const int t = job / nch, nt = (p.w_rows + 63) / 64;
+      const bool second = t >= nt;
+      if (t >= (p.W2 ? 2 * nt : nt)) return;
+      pack_chunk<(int)T, SP>(p, second ? p.W2 : p.W, p.w_row0 / 64 + (second ? t - nt : t), job - t * nch);
     }
   } else {
     const int job = ((int)blockIdx.x - p.w_groups) * 4 + wave;
@@ -177,7 +183,9 @@ __global__ __launch_bounds__(256) void pack_kernel(PackArgs p) {
 // on both sides of it, and no read waits for its own stage's copy.
 // The activations are the A operand (rows of D): a lane then holds one weight row's column of D,
 // and a store instruction writes two whole 128-byte runs of two output rows.
-template <int BM, int BN, int WM, int WN, int KK, int NB, bool SP>
+// SW: the SwiGLU epilogue. The weights are the A operand, so a lane holds one activation row and runs of
+// four consecutive weight rows, and writes h as 8-byte halves of the next GEMM's fragment units.
+template <int BM, int BN, int WM, int WN, int KK, int NB, bool SP, bool SW>
 __global__ __launch_bounds__(WM* WN * 64) void packed_gemm_kernel(PackedGemmArgs p) {
   constexpr int NWAVE = WM * WN;
   constexpr int TM = BM / WM / 32, TN = BN / WN / 32;
@@ -253,8 +261,9 @@ __global__ __launch_bounds__(WM* WN * 64) void packed_gemm_kernel(PackedGemmArgs
   // MFMA i of a stage: per k step the w_hi x_hi products, then (f32 mode) w_hi x_lo and w_lo x_hi
   auto mma = [&](const Ops& o, int i) {
     const int kk = i / (NM / KK), term = i / (TM * TN) % (SP ? 3 : 1), m = i / TN % TM, n = i % TN;
-    acc[n][m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(o.x[kk][SP && term == 1][n], o.w[kk][SP && term == 2][m],
-                                                        acc[n][m], 0, 0, 0);
+    const bf16x8_t x = o.x[kk][SP && term == 1][n], w = o.w[kk][SP && term == 2][m];
+    acc[n][m] = SW ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(w, x, acc[n][m], 0, 0, 0)
+                   : __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, w, acc[n][m], 0, 0, 0);
   };
   auto sync = [&]() {
     asm volatile("" ::: "memory");
@@ -299,6 +308,49 @@ __global__ __launch_bounds__(WM* WN * 64) void packed_gemm_kernel(PackedGemmArgs
   }
   wait_copies<0>();                            // no copy into LDS outlives the workgroup
 
+  if constexpr (SW) {
+    static_assert(TM % 2 == 0, "whole gate / up pairs per wave");
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int x = BN * ntile + BN / WN * wn + 32 * j + (lane & 31);
+      if (x >= p.N) continue;
+#pragma unroll
+      for (int i = 0; i < TM; i += 2) {
+        const int k0 = (BM * mtile + BM / WM * wm + 32 * i) / 2;   // h columns k0 .. k0 + 31
+        if (2 * k0 >= p.m) continue;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          bf16x4_t hi, lo;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float v = silu_mul(acc[j][i][4 * q + e], acc[j][i + 1][4 * q + e]);
+            hi[e] = (__bf16)v;
+            lo[e] = (__bf16)(v - (float)hi[e]);
+          }
+          uint8_t* d = p.Hp + unit_off(x, k0 + 8 * q, p.KSh) + 8 * (lane >> 5);
+          *reinterpret_cast<bf16x4_t*>(d) = hi;
+          if constexpr (SP) *reinterpret_cast<bf16x4_t*>(d + p.h_lo) = lo;
+        }
+      }
+    }
+    return;
+  }
+  if (p.add) {                             // (splits 1)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        const int w = BM * mtile + BM / WM * wm + 32 * i + (lane & 31);
+        if (w >= p.m) continue;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int x = BN * ntile + BN / WN * wn + 32 * j + 4 * (lane >> 5) + 8 * (r >> 2) + (r & 3);
+          const size_t o = (size_t)x * p.ldy + w;
+          if (x < p.N) p.Y[o] = p.add[o] + acc[j][i][r];
+        }
+      }
+    return;
+  }
   float* Y = p.splits > 1 ? p.partial + (size_t)split * p.split_stride : p.Y;
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
@@ -320,11 +372,11 @@ __global__ __launch_bounds__(WM* WN * 64) void packed_gemm_kernel(PackedGemmArgs
   }
 }
 
-template <int BM, int BN, int WM, int WN, int KK, int NB, bool SP>
+template <int BM, int BN, int WM, int WN, int KK, int NB, bool SP, bool SW = false>
 hipError_t launch_shape(const PackedGemmArgs& a, hipStream_t s) {
   const int total = ((a.m + BM - 1) / BM) * ((a.N + BN - 1) / BN) * a.splits;
   const int grid = (total + 7) / 8 * 8;
-  hipLaunchKernelGGL((packed_gemm_kernel<BM, BN, WM, WN, KK, NB, SP>), dim3((unsigned)grid), dim3(WM * WN * 64), 0, s, a);
+  hipLaunchKernelGGL((packed_gemm_kernel<BM, BN, WM, WN, KK, NB, SP, SW>), dim3((unsigned)grid), dim3(WM * WN * 64), 0, s, a);
   return hipGetLastError();
 }
 
@@ -342,6 +394,7 @@ hipError_t launch_pack(uint32_t type, PackArgs a, bool sp, hipStream_t s) {
   long wjobs;
   if (type == 0 || type == 1 || type == 30) wjobs = (long)((a.w_rows + 31) / 32) * kcs;
   else wjobs = (long)((a.w_rows + 63) / 64) * a.KB * (type == T_Q4_K || type == T_Q5_K || type == T_Q6_K ? 8 : 1);
+  if (a.W2) wjobs *= 2;
   const long xjobs = (long)((a.x_rows + 31) / 32) * kcs;
   a.w_groups = (int)((wjobs + 3) / 4);
   const unsigned grid = (unsigned)(a.w_groups + (xjobs + 3) / 4);
@@ -361,6 +414,22 @@ hipError_t launch_pack(uint32_t type, PackArgs a, bool sp, hipStream_t s) {
 }
 
 hipError_t launch_packed_gemm(const PackedGemmArgs& a, PackedTile tile, bool sp, hipStream_t s) {
+  if (a.Hp) {
+    if (a.splits != 1) return hipErrorInvalidValue;
+    if (sp) {
+      switch (tile) {
+        case PackedTile::k256x128: return launch_shape<256, 128, 4, 2, 2, 3, true, true>(a, s);
+        case PackedTile::k128x128: return launch_shape<128, 128, 2, 2, 2, 4, true, true>(a, s);
+        case PackedTile::k128x64: return launch_shape<128, 64, 2, 2, 2, 3, true, true>(a, s);
+        default: return hipErrorInvalidValue;
+      }
+    }
+    switch (tile) {
+      case PackedTile::k256x256: return launch_shape<256, 256, 2, 4, 2, 4, false, true>(a, s);
+      case PackedTile::k128x128: return launch_shape<128, 128, 2, 2, 2, 4, false, true>(a, s);
+      default: return hipErrorInvalidValue;
+    }
+  }
   if (sp) {
     switch (tile) {
       case PackedTile::k256x128: return launch_shape<256, 128, 4, 2, 2, 3, true>(a, s);
@@ -378,7 +447,7 @@ hipError_t launch_packed_gemm(const PackedGemmArgs& a, PackedTile tile, bool sp,
   }
 }
 
-PackedPlan plan_packed(int m, int rows, int K, bool sp) {
+PackedPlan plan_packed(int m, int rows, int K, bool sp, bool pairs) {
   // The fullest CU's tiles times the stages of one, at the measured time of a stage (32 k; us, on
   // 961 x 4864 x 896, 961 x 896 x 4864, 4096^3 and 2048 x 14336 x 4096), plus the bytes of the
   // outputs and, for K slices, of the partial tiles and their reduce at 4 TB/s and its launch.
@@ -393,8 +462,9 @@ PackedPlan plan_packed(int m, int rows, int K, bool sp) {
   PackedPlan best;
   double best_us = 1e30;
   for (int i = 0; i < ns; ++i) {
+    if (pairs && sh[i].t == PackedTile::k192x128) continue;   // three 32-row groups per wave
     const long tiles = (long)((m + sh[i].bm - 1) / sh[i].bm) * ((rows + sh[i].bn - 1) / sh[i].bn);
-    for (int sp_n = 1; sp_n <= 8; ++sp_n) {
+    for (int sp_n = 1; sp_n <= (pairs ? 1 : 8); ++sp_n) {
       const int per = (steps + sp_n - 1) / sp_n;
       if (sp_n > 1 && (per < 4 || (steps + per - 1) / per != sp_n || (double)sp_n * rows * m * 4 > (32 << 20))) continue;
       double us = (double)((tiles * sp_n + 255) / 256) * per * sh[i].us + out_us * sp_n;

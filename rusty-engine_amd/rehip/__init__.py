@@ -42,7 +42,8 @@ EXPORTS = ("re_init", "re_last_error", "re_version", "re_row_bytes", "re_tiled_b
            "re_qmat_dequant_dev", "re_dequant", "re_moe_create", "re_moe_destroy", "re_moe_forward",
            "re_moe_forward_dev", "re_qmat_matvec_ex_dev", "re_rmsnorm_dev", "re_rope_dev", "re_kv_append_dev",
            "re_attention_dev", "re_add_dev", "re_swiglu_dev", "re_argmax_dev", "re_embed_dev", "re_pos_add_dev",
-           "re_ffn_create", "re_ffn_destroy", "re_ffn_forward_dev", "re_attention_work_bytes",
+           "re_ffn_create", "re_ffn_destroy", "re_ffn_forward_dev", "re_ffn_block_work_bytes", "re_ffn_block_dev",
+           "re_attention_work_bytes",
            "re_qkv_rope_append_dev", "re_decode_advance_dev",
            "re_qmat_create_stacked", "re_qmat_count", "re_qmat_matvec_stacked_dev", "re_moe_router_logits_dev",
            "re_moe_route_dev", "re_moe_forward_routed_dev", "re_moe_layer_dev",
@@ -131,6 +132,9 @@ def lib() -> C.CDLL:
         L.re_ffn_destroy.argtypes = [_vp]
         L.re_ffn_destroy.restype = None
         L.re_ffn_forward_dev.argtypes = [_vp, _vp, _vp, C.c_float, _vp, _vp]
+        L.re_ffn_block_work_bytes.argtypes = [_vp, _vp, _sz]
+        L.re_ffn_block_work_bytes.restype = _sz
+        L.re_ffn_block_dev.argtypes = [_vp, _vp, _vp, _sz, _vp, _vp, _vp, _sz, C.c_int, _vp]
         L.re_gguf_open.argtypes = [C.c_char_p, C.POINTER(_vp)]
         L.re_gguf_close.argtypes = [_vp]
         L.re_gguf_close.restype = None
@@ -463,6 +467,15 @@ class Ffn:
     def forward_dev(self, x_dev, h_dev, norm_w=None, eps=0.0, stream=None) -> None:
         _check(lib().re_ffn_forward_dev(self._h, _dev_ptr(x_dev), _p(norm_w), eps, _dev_ptr(h_dev),
                                         _stream_ptr(stream)))
+
+    def block_work_bytes(self, down: "QMat", rows: int) -> int:
+        return int(lib().re_ffn_block_work_bytes(self._h, down._h, rows))
+
+    def block_dev(self, down: "QMat", x_dev, rows: int, y_dev, work_dev, work_bytes: int, mode: int = MODE_F32,
+                  add=None, stream=None) -> None:
+        """y = add + down(silu(gate x) * up x) over `rows` rows (add may be y)."""
+        _check(lib().re_ffn_block_dev(self._h, down._h, _dev_ptr(x_dev), rows, _p(add), _dev_ptr(y_dev),
+                                      _dev_ptr(work_dev), work_bytes, mode, _stream_ptr(stream)))
 
     def close(self) -> None:
         if self._h:

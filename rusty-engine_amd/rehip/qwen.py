@@ -539,10 +539,10 @@ class DeviceDecoder:
         self.qkv = B(cap * (d + 2 * kv) * 4)
         self.qb = B(cap * d * 4)
         self.ctx = B(cap * d * 4)
-        self.ob = B(cap * g.d_ff * 4)       # o / down outputs of the prefill
-        self.gb = B(cap * g.d_ff * 4)
-        self.ub = B(cap * g.d_ff * 4)
-        self.hb = B(cap * g.d_ff * 4)
+        self.ob = B(cap * d * 4)            # o outputs of the prefill
+        self.hb = B(g.d_ff * 4)             # the FFN of one decode row
+        self.ffn_bytes = max(blk["ffn"].block_work_bytes(blk["down"], cap) for blk in self.blocks) if self.blocks else 256
+        self.ffn_work = B(self.ffn_bytes)
         self.logits_buf = B(mb.n_vocab * 4)
         self.work_bytes = attention_work_bytes(8, g.n_heads, hd, max_seq)
         self.work = B(self.work_bytes)
@@ -631,7 +631,7 @@ class DeviceDecoder:
     # -- API -------------------------------------------------------------------------------
     def prefill(self, prompt) -> int:
         """Batched prefill of the prompt (runner.rs:236-260); returns the first greedy token."""
-        from . import add_dev, embed_dev, rmsnorm_dev, swiglu_dev
+        from . import add_dev, embed_dev, rmsnorm_dev
         g, s, m = self.g, self.stream, self.mode
         d = g.d_model
         prompt = np.asarray(prompt, np.int32)
@@ -650,11 +650,8 @@ class DeviceDecoder:
             blk["o"].matmul_dev(self.ctx, rows, self.ob, m, stream=s)
             add_dev(self.x, self.ob, rows * d, rows * d, self.x, s)
             rmsnorm_dev(self.x, blk["ffn_norm"], rows, d, g.rms_eps, self.n, s)
-            blk["gate"].matmul_dev(self.n, rows, self.gb, m, stream=s)
-            blk["up"].matmul_dev(self.n, rows, self.ub, m, stream=s)
-            swiglu_dev(self.gb, self.ub, self.hb, rows * g.d_ff, s)
-            blk["down"].matmul_dev(self.hb, rows, self.ob, m, stream=s)
-            add_dev(self.x, self.ob, rows * d, rows * d, self.x, s)
+            blk["ffn"].block_dev(blk["down"], self.n, rows, self.x, self.ffn_work, self.ffn_bytes, m, add=self.x,
+                                 stream=s)
         self._head_and_advance(_Offset(self.x, (rows - 1) * d * 4), rows)
         self.seq_len += rows
         self.stream.synchronize()
