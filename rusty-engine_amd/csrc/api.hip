@@ -657,10 +657,25 @@ int packed_enqueue(const PackedCall& c, const float* d_x, float* d_y, void* ws, 
   return RE_OK;
 }
 
+// Grow the matrix's K-split partials for the GEMM that a captured call of this shape takes, as an eager
+// call of it would (a graph captured after an eager call on packed operands otherwise ran unsplit: Q6_K
+// 896 x 4864, 961 rows, 106 instead of 29 us). Out of memory only costs the split.
+void warm_partials(re_qmat* q, size_t rows, int mode) {
+  int splits = 1;
+  if (q->dense) {
+    splits = dense_mma_splits((int)q->g.m, (int)q->g.n, (int)rows);
+    if ((size_t)splits * rows * q->g.m * sizeof(float) > (32u << 20)) return;
+  } else {
+    splits = plan_gemm((int)q->g.m, (int)rows, (int)q->g.n, mode == RE_MODE_F32 ? kGemmModeSplit : mode).splits;
+  }
+  const size_t need = (size_t)splits * rows * q->g.m * sizeof(float);
+  if (splits > 1 && need > q->spart.cap) (void)q->spart.ensure(need);
+}
+
 // The call on packed operands, in a workspace of the GPU's; *ran = false (and nothing enqueued) where
 // it cannot be had: under stream capture (a replayed graph would use the shared buffers outside
 // their ordering), no buffer left, or out of memory.
-int packed_shared(const PackedCall& c, const float* d_x, float* d_y, hipStream_t s, bool* ran) {
+int packed_shared(re_qmat* q, const PackedCall& c, const float* d_x, float* d_y, int mode, hipStream_t s, bool* ran) {
   *ran = false;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   HIP_TRY(hipStreamIsCapturing(s, &cs));
@@ -668,6 +683,7 @@ int packed_shared(const PackedCall& c, const float* d_x, float* d_y, hipStream_t
   int dev = 0;
   HIP_TRY(hipGetDevice(&dev));
   if (dev < 0 || dev >= kPackedDevices) return RE_OK;
+  warm_partials(q, c.rows, mode);
   const size_t bytes = c.want(kPackedWsBytes);
   std::lock_guard<std::mutex> lk(g_packed_mu);
   PackedSlot* sl = packed_slot(g_packed[dev], bytes, s);
@@ -694,7 +710,7 @@ bool packed_ffn_pays(size_t ff, size_t K, size_t rows, bool sp) {
 // in memory in f32 and x is packed once; the residual is added in the down GEMM's epilogue or reduce.
 // Weights larger than the workspace go in pieces. 961-row prefill of 24 layers (896 x 4864): 4271 -> 3629 us.
 // *ran = false (and nothing enqueued) where the rule or the workspace says no.
-int packed_ffn(const re_qmat* gate, const re_qmat* up, const re_qmat* down, const float* d_x, size_t rows,
+int packed_ffn(re_qmat* gate, re_qmat* up, re_qmat* down, const float* d_x, size_t rows,
                const float* d_add, float* d_y, int mode, hipStream_t s, bool* ran) {
   *ran = false;
   const size_t ff = gate->g.m, d = down->g.m;
@@ -727,6 +743,7 @@ int packed_ffn(const re_qmat* gate, const re_qmat* up, const re_qmat* down, cons
   int dev = 0;
   HIP_TRY(hipGetDevice(&dev));
   if (dev < 0 || dev >= kPackedDevices) return RE_OK;
+  for (re_qmat* q : {gate, up, down}) warm_partials(q, rows, mode);
   std::lock_guard<std::mutex> lk(g_packed_mu);
   PackedSlot* sl = packed_slot(g_packed[dev], total, s);
   if (!sl) return RE_OK;
@@ -865,7 +882,7 @@ int gemm_enqueue(re_qmat* q, const float* d_x, size_t rows, float* d_y, int mode
   if (packed_call(q->g.type, q->d_w, q->g.m, q->g.n, q->g.kb, d_x, rows, mode, &pc)) {
     if (fixed_partial) return packed_enqueue(pc, d_x, d_y, fixed_partial, fixed_cap, s);
     bool ran = false;
-    const int rc = packed_shared(pc, d_x, d_y, s, &ran);
+    const int rc = packed_shared(q, pc, d_x, d_y, mode, s, &ran);
     if (rc || ran) return rc;
   }
   // f32 mode on bf16 MFMAs with split operands (REHIP_GEMM_SP=0: the f32 MFMA tiles)
@@ -1194,7 +1211,7 @@ int re_qmat_matmul_dev(re_qmat* q, const float* d_x, size_t rows, float* d_y, in
     PackedCall pc;
     if (dense_packed(q, d_x, rows, mode, &pc)) {
       bool ran = false;
-      const int rc = packed_shared(pc, d_x, d_y, s, &ran);
+      const int rc = packed_shared(q, pc, d_x, d_y, mode, s, &ran);
       if (rc || ran) return rc;
     }
     int splits = 1;

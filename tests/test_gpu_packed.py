@@ -132,3 +132,27 @@ def test_streams_and_capture():
         s.destroy()
     for q in qs:
         q.close()
+
+
+def test_capture_after_eager_call_keeps_its_slices():
+    """A graph captured after an eager call (which ran on packed operands) takes the tiled GEMM with its
+    K slices: the bits of a call that never packs."""
+    m, n, rows = 896, 4864, 400
+    rng = np.random.default_rng(8)
+    w, dx = weights(rng, rehip.Q6_K, m, n), B.from_array(synth.activations(rng, rows, n))
+    got = []
+    for packed in (True, False):
+        q = rehip.QMat.from_bytes(rehip.Q6_K, w, m, n)
+        s, y = hip.Stream(), B(rows * m * 4)
+        with pytest.MonkeyPatch.context() as mp:
+            if not packed:
+                mp.setenv("REHIP_GEMM_PACKED", "0")
+            q.matmul_dev(dx, rows, y, rehip.MODE_BF16, stream=s)
+            g = hip.Graph(s, lambda: q.matmul_dev(dx, rows, y, rehip.MODE_BF16, stream=s))
+        g.launch()
+        hip.synchronize()
+        got.append(y.download(np.float32, rows * m))
+        g.destroy()
+        s.destroy()
+        q.close()
+    assert np.array_equal(got[0], got[1])
