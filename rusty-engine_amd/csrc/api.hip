@@ -708,7 +708,7 @@ bool packed_ffn_pays(size_t ff, size_t K, size_t rows, bool sp) {
 // groups and multiplied by one GEMM whose epilogue writes h as the down projection's packed
 // activations (the rounding that packing the f32 h would give), so neither gate, up nor h are ever
 // in memory in f32 and x is packed once; the residual is added in the down GEMM's epilogue or reduce.
-// Weights larger than the workspace go in pieces. 961-row prefill of 24 layers (896 x 4864): 4271 -> 3629 us.
+// Weights larger than the workspace go in pieces. 961-row prefill of 24 layers (896 x 4864): 4271 -> 3520 .. 3660 us.
 // *ran = false (and nothing enqueued) where the rule or the workspace says no.
 int packed_ffn(re_qmat* gate, re_qmat* up, re_qmat* down, const float* d_x, size_t rows,
                const float* d_add, float* d_y, int mode, hipStream_t s, bool* ran) {
