@@ -112,17 +112,18 @@ __device__ __forceinline__ void pack_rows(const void* src, int rows, int K, int 
 }
 
 // One wave packs one 32-quant chunk of a slab's 64 rows (lane = row): the four units of the
-// chunk's two 16-element runs.
+// chunk's two 16-element runs. second: of W2 (which may be the same matrix as W).
 template <int T, bool SP>
-__device__ __forceinline__ void pack_chunk(const PackArgs& p, const void* W, int tile, int c) {
+__device__ __forceinline__ void pack_chunk(const PackArgs& p, bool second, int tile, int c) {
   using B = Blk<T>;
+  const void* W = second ? p.W2 : p.W;
   const int lane = threadIdx.x & 63;
   const int kb = c / B::NCH, cc = c - kb * B::NCH;
   const uint8_t* slab = (const uint8_t*)W + ((size_t)tile * p.KB + kb) * B::SLAB;
   int row = 64 * tile + lane - p.w_row0;
   if (p.W2) {
     if (row >= p.w_rows) return;          // (the other matrix's groups would follow)
-    row = 2 * row - (row & 31) + (W == p.W2 ? 32 : 0);
+    row = 2 * row - (row & 31) + (second ? 32 : 0);
   }
   Run a, b;
   B::chunk(slab, lane, cc, a, b);
@@ -165,7 +166,7 @@ __global__ __launch_bounds__(256) void pack_kernel(PackArgs p) {
       const int t = job / nch, nt = (p.w_rows + 63) / 64;
       const bool second = t >= nt;
       if (t >= (p.W2 ? 2 * nt : nt)) return;
-      pack_chunk<(int)T, SP>(p, second ? p.W2 : p.W, p.w_row0 / 64 + (second ? t - nt : t), job - t * nch);
+      pack_chunk<(int)T, SP>(p, second, p.w_row0 / 64 + (second ? t - nt : t), job - t * nch);
     }
   } else {
     const int job = ((int)blockIdx.x - p.w_groups) * 4 + wave;

@@ -94,6 +94,28 @@ def test_equals_separate_calls(mode, rows):
         m.close()
 
 
+@pytest.mark.parametrize("mode", MODES)
+def test_one_matrix_as_gate_and_up(mode):
+    """The packed path against the separate calls where gate and up are one matrix, after a call on other
+    weights that leaves its packed groups in the shared workspace."""
+    d, ff, rows = 256, 512, 150
+    rng = np.random.default_rng(11)
+    w = matrices(rng, rehip.Q4_K, rehip.Q6_K, d, ff)
+    q = [rehip.QMat.from_bytes(t, b, *s) for t, b, s in zip((rehip.Q4_K, rehip.Q4_K, rehip.Q6_K), w,
+                                                            ((ff, d), (ff, d), (d, ff)))]
+    x = (0.1 * synth.activations(rng, rows, d)).astype(np.float32)
+    got = []
+    for knob in ("2", "0"):
+        with pytest.MonkeyPatch.context() as mp:
+            mp.setenv("REHIP_GEMM_PACKED", knob)
+            block(q, x, rows, d, mode)
+            got.append(block([q[1], q[1], q[2]], x, rows, d, mode))
+    # products in another order of sums: an h may round to bf16 the other way (2^-8 of it)
+    assert np.linalg.norm(got[0] - got[1]) <= (2.0 ** -8 if mode == rehip.MODE_BF16 else 2e-5) * np.linalg.norm(got[1])
+    for m in q:
+        m.close()
+
+
 def test_errors():
     rng = np.random.default_rng(1)
     w = matrices(rng, rehip.Q4_0, rehip.Q4_0, 64, 96)
