@@ -88,7 +88,10 @@ int re_qmat_matvec(re_qmat *q, const float *x, float *y);
  * the GEMV; otherwise the MFMA GEMM in the given mode. */
 int re_qmat_matmul(re_qmat *q, const float *x, size_t rows, float *y, int mode);
 
-/* Device-pointer variants; `stream` is a hipStream_t (NULL = default stream). */
+/* Device-pointer variants; `stream` is a hipStream_t (NULL = default stream). re_qmat_matmul_dev
+ * allocates on first use: up to 32 MiB per matrix for K-split partial tiles and, for the calls of many
+ * rows that run on packed bf16 operands, workspaces shared by all matrices of a GPU (at most 4 of
+ * 64 .. 512 MiB, ordered between streams by events, freed with the last matrix). */
 int re_qmat_matvec_dev(re_qmat *q, const float *d_x, float *d_y, void *stream);
 int re_qmat_matmul_dev(re_qmat *q, const float *d_x, size_t rows, float *d_y, int mode,
                        void *stream);
@@ -99,9 +102,9 @@ int re_qmat_matmul_dev(re_qmat *q, const float *d_x, size_t rows, float *d_y, in
  * and results as re_qmat_matmul_dev (operands larger than the scratch are packed and multiplied in
  * pieces). A plan whose partials exceed the scratch fails with RE_ERR_SIZE (the planned splits of
  * every shape fit: the planner caps partial tiles at 32 MiB). The scratch
- * is shared by every call on a GPU. Outside stream capture, a call on a different stream than the
- * previous call on that GPU first waits for the previous call's launches (an event set up once per
- * device), so calls from several streams or threads stay ordered. Inside stream capture no
+ * is shared by every call on a GPU. Outside stream capture, a call first waits for the launches of the
+ * previous call on that GPU (an event set up once per device), so calls from several streams or threads
+ * stay ordered. Inside stream capture no
  * ordering is added: replays of captured graphs that use the scratch must not overlap in time. */
 int re_qmat_matmul_noalloc_dev(re_qmat *q, const float *d_x, size_t rows, float *d_y, int mode, void *stream);
 /* Dequantize the resident weights to d_out[m x n] f32, bit-exact with quant::dequant. */

@@ -448,82 +448,95 @@ int gemv_enqueue(re_qmat* q, const float* d_x, float* d_y, hipStream_t s, const 
 // ---- GEMM over packed bf16 operands (packed.hip) ---------------------------------------------
 // The packed operands live in a workspace only while the call's launches run: up to kPackedSlots
 // buffers per GPU, shared by every matrix (a buffer per matrix would hold another 2-4 bytes per
-// weight). A buffer belongs to one stream at a time, so the stream orders its uses and a call pays
-// for no event (one recorded per call left the GPU idle for 1-4 us). A stream gives its buffer back
-// when a host-pointer call has synchronized it; the buffer of a stream that no longer exists is
-// freed (hipFree waits for the device) and allocated anew. A call that finds no buffer runs on the
-// tiled GEMM. All are freed with the last matrix. (A new stream may get a destroyed stream's handle;
-// the runtime has finished the old stream's work by then.)
+// weight), freed with the last matrix. A buffer's event is carried by the last launch of the call that
+// used it, and the next call waits for it whatever its stream (equal handles prove nothing: a new stream
+// may get the handle of a destroyed one whose work is still in flight). The event rides on the kernel's
+// own completion signal, without a system-scope release: 0.03 us a call, where a recorded one left
+// the GPU idle for 2.9 us (1.1 without the release). A call takes the buffer that its stream's handle
+// used last, else an unused one, else the one used longest ago.
 constexpr size_t kPackedWsBytes = 512u << 20;    // largest workspace; larger operands run in pieces
-constexpr int kPackedSlots = 8, kPackedDevices = 64;
+constexpr size_t kPackedMinBytes = 64u << 20;    // smallest; a buffer at least doubles when it grows
+constexpr int kPackedSlots = 4, kPackedDevices = 64;
 struct PackedSlot {
   void* p = nullptr;
   size_t cap = 0;
-  bool owned = false;                             // by `stream`
-  hipStream_t stream = nullptr;
+  hipEvent_t done = nullptr;                      // of the last call
+  bool used = false;
+  hipStream_t last = nullptr;
+  unsigned long long turn = 0;                    // when it was last used
 };
-std::mutex g_packed_mu;
-PackedSlot g_packed[kPackedDevices][kPackedSlots];
+struct PackedPool {
+  std::mutex mu;
+  PackedSlot slots[kPackedSlots];
+  unsigned long long turns = 0;
+};
+PackedPool g_packed[kPackedDevices];
+std::mutex g_packed_users_mu;
 long g_packed_users = 0;                          // live matrices
 
 void packed_user(int delta) {
-  std::lock_guard<std::mutex> lk(g_packed_mu);
+  std::lock_guard<std::mutex> lk(g_packed_users_mu);
   g_packed_users += delta;
   if (g_packed_users > 0) return;
-  for (auto& dev : g_packed)
-    for (PackedSlot& sl : dev) {
+  for (PackedPool& pool : g_packed) {
+    std::lock_guard<std::mutex> plk(pool.mu);
+    for (PackedSlot& sl : pool.slots) {
       if (sl.p) (void)hipFree(sl.p);              // waits for the work that uses it
+      if (sl.done) (void)hipEventDestroy(sl.done);
       sl = PackedSlot{};
     }
-}
-
-// the stream has been synchronized (or is about to go): its buffer is idle
-void packed_idle(hipStream_t s) {
-  std::lock_guard<std::mutex> lk(g_packed_mu);
-  for (auto& dev : g_packed)
-    for (PackedSlot& sl : dev)
-      if (sl.owned && sl.stream == s) sl.owned = false;
-}
-
-// whether the handle still names a stream
-bool stream_lives(hipStream_t s) {
-  unsigned flags = 0;
-  if (!s || hipStreamGetFlags(s, &flags) == hipSuccess) return true;
-  (void)hipGetLastError();
-  return false;
-}
-
-// A buffer of `bytes` for stream s (g_packed_mu held), or nullptr.
-PackedSlot* packed_slot(PackedSlot* slots, size_t bytes, hipStream_t s) {
-  if (s == hipStreamPerThread) return nullptr;    // one handle, but a stream per thread
-  PackedSlot* pick = nullptr;
-  int score = 0;
-  for (int i = 0; i < kPackedSlots; ++i) {
-    PackedSlot& sl = slots[i];
-    const int sc = sl.owned ? (sl.stream == s ? 4 : 0) : !sl.p ? 2 : sl.cap >= bytes ? 3 : 1;
-    if (sc > score) { score = sc; pick = &sl; }
   }
-  for (int i = 0; i < kPackedSlots && !pick; ++i) {
-    if (stream_lives(slots[i].stream)) continue;
-    pick = &slots[i];                             // its stream is gone
-    (void)hipFree(pick->p);
+}
+
+// A buffer of `bytes` for stream s (pool.mu held), or nullptr.
+PackedSlot* packed_slot(PackedPool& pool, size_t bytes, hipStream_t s) {
+  PackedSlot* pick = nullptr;
+  for (PackedSlot& sl : pool.slots) {
+    auto rank = [&](const PackedSlot& x) { return x.used ? (x.last == s ? 2 : 0) : 1; };
+    if (!pick || rank(sl) > rank(*pick) || (rank(sl) == rank(*pick) && sl.turn < pick->turn)) pick = &sl;
+  }
+  if (pick->cap < bytes) {
+    const size_t want = std::max(bytes, std::min(kPackedWsBytes, std::max(kPackedMinBytes, 2 * pick->cap)));
+    if (pick->p) (void)hipFree(pick->p);          // waits for the device
     pick->p = nullptr;
     pick->cap = 0;
-  }
-  if (!pick) return nullptr;
-  if (pick->cap < bytes) {
-    if (pick->p) (void)hipFree(pick->p);
-    *pick = PackedSlot{};
-    if (hipMalloc(&pick->p, bytes) != hipSuccess) {
+    pick->used = false;
+    if ((!pick->done &&
+         hipEventCreateWithFlags(&pick->done, hipEventDisableTiming | hipEventDisableSystemFence) != hipSuccess) ||
+        hipMalloc(&pick->p, want) != hipSuccess) {
       (void)hipGetLastError();
       pick->p = nullptr;
       return nullptr;
     }
-    pick->cap = bytes;
+    pick->cap = want;
   }
-  pick->owned = true;
-  pick->stream = s;
   return pick;
+}
+
+// Runs enqueue(buffer, event) with a buffer of `bytes` of the current GPU's; *ran = false (and nothing
+// enqueued) where none can be had: under stream capture (a replayed graph would use the shared buffers
+// outside their ordering) or out of memory. The last launch of enqueue has to carry the event.
+template <typename F>
+int with_packed_slot(size_t bytes, hipStream_t s, bool* ran, F&& enqueue) {
+  *ran = false;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  HIP_TRY(hipStreamIsCapturing(s, &cs));
+  if (cs != hipStreamCaptureStatusNone) return RE_OK;
+  int dev = 0;
+  HIP_TRY(hipGetDevice(&dev));
+  if (dev < 0 || dev >= kPackedDevices) return RE_OK;
+  PackedPool& pool = g_packed[dev];
+  std::lock_guard<std::mutex> lk(pool.mu);        // (also keeps the launches of one call together)
+  PackedSlot* sl = packed_slot(pool, bytes, s);
+  if (!sl) return RE_OK;
+  if (sl->used) HIP_TRY(hipStreamWaitEvent(s, sl->done, 0));
+  *ran = true;
+  sl->used = true;
+  sl->last = s;
+  sl->turn = ++pool.turns;
+  const int rc = enqueue(sl->p, sl->done);
+  if (rc) (void)hipEventRecord(sl->done, s);      // after what was enqueued before the error
+  return rc;
 }
 
 struct PackedCall {
@@ -603,7 +616,9 @@ bool dense_packed(const re_qmat* q, const float* d_x, size_t rows, int mode, Pac
          packed_call(q->g.type, q->d_w, q->g.m, q->g.n, 0, d_x, rows, mode, c);
 }
 
-int packed_enqueue(const PackedCall& c, const float* d_x, float* d_y, void* ws, size_t ws_bytes, hipStream_t s) {
+// done: carried by the last launch (nullptr: none)
+int packed_enqueue(const PackedCall& c, const float* d_x, float* d_y, void* ws, size_t ws_bytes, hipStream_t s,
+                   hipEvent_t done = nullptr) {
   const size_t rb = c.row_bytes(), part = c.partial_bytes(), avail = ws_bytes - part;
   const size_t mp = PackedCall::pad(c.m), np = PackedCall::pad(c.rows);
   size_t mc = mp, nc = np;                       // rows of each operand packed at a time
@@ -650,10 +665,11 @@ int packed_enqueue(const PackedCall& c, const float* d_x, float* d_y, void* ws, 
       a.ldy = c.m;
       a.splits = c.plan.splits;
       a.steps_per_split = c.plan.steps_per_split;
-      HIP_TRY(launch_packed_gemm(a, c.plan.tile, c.sp, s));
+      const bool last = n0 + nc >= (size_t)c.rows && m0 + mc >= (size_t)c.m;
+      HIP_TRY(launch_packed_gemm(a, c.plan.tile, c.sp, s, last && !partial ? done : nullptr));
     }
   }
-  if (partial) HIP_TRY(launch_gemm_reduce(partial, d_y, (size_t)c.rows * c.m, c.plan.splits, s));
+  if (partial) HIP_TRY(launch_gemm_reduce(partial, d_y, (size_t)c.rows * c.m, c.plan.splits, s, nullptr, done));
   return RE_OK;
 }
 
@@ -672,24 +688,13 @@ void warm_partials(re_qmat* q, size_t rows, int mode) {
   if (splits > 1 && need > q->spart.cap) (void)q->spart.ensure(need);
 }
 
-// The call on packed operands, in a workspace of the GPU's; *ran = false (and nothing enqueued) where
-// it cannot be had: under stream capture (a replayed graph would use the shared buffers outside
-// their ordering), no buffer left, or out of memory.
+// The call on packed operands, in a workspace of the GPU's (*ran as in with_packed_slot).
 int packed_shared(re_qmat* q, const PackedCall& c, const float* d_x, float* d_y, int mode, hipStream_t s, bool* ran) {
-  *ran = false;
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  HIP_TRY(hipStreamIsCapturing(s, &cs));
-  if (cs != hipStreamCaptureStatusNone) return RE_OK;
-  int dev = 0;
-  HIP_TRY(hipGetDevice(&dev));
-  if (dev < 0 || dev >= kPackedDevices) return RE_OK;
-  warm_partials(q, c.rows, mode);
   const size_t bytes = c.want(kPackedWsBytes);
-  std::lock_guard<std::mutex> lk(g_packed_mu);
-  PackedSlot* sl = packed_slot(g_packed[dev], bytes, s);
-  if (!sl) return RE_OK;
-  *ran = true;
-  return packed_enqueue(c, d_x, d_y, sl->p, bytes, s);
+  return with_packed_slot(bytes, s, ran, [&](void* ws, hipEvent_t done) {
+    warm_partials(q, c.rows, mode);
+    return packed_enqueue(c, d_x, d_y, ws, bytes, s, done);
+  });
 }
 
 // Whether a whole FFN on packed operands beats its separate calls (each by its own best route), by shape
@@ -737,86 +742,78 @@ int packed_ffn(re_qmat* gate, re_qmat* up, re_qmat* down, const float* d_x, size
   const size_t fc = piece(2 * ff, rb1) / 2, dc = piece(d, rb2);   // fc rows of gate and fc of up
   if (fc == 0 || dc == 0) return RE_OK;
   const size_t total = fixed + region;
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  HIP_TRY(hipStreamIsCapturing(s, &cs));
-  if (cs != hipStreamCaptureStatusNone) return RE_OK;
-  int dev = 0;
-  HIP_TRY(hipGetDevice(&dev));
-  if (dev < 0 || dev >= kPackedDevices) return RE_OK;
-  for (re_qmat* q : {gate, up, down}) warm_partials(q, rows, mode);
-  std::lock_guard<std::mutex> lk(g_packed_mu);
-  PackedSlot* sl = packed_slot(g_packed[dev], total, s);
-  if (!sl) return RE_OK;
-  *ran = true;
-  uint8_t* ws = (uint8_t*)sl->p;
-  uint8_t *xp = ws + part, *hp = xp + xb, *wp = hp + hb;
-  const int planes = sp ? 2 : 1, KS1 = (c1.K + 31) / 32 * 2, KS2 = (c2.K + 31) / 32 * 2;
-  for (size_t f0 = 0; f0 < ff; f0 += fc) {      // fc is a multiple of 128: whole slabs and h fragments
-    PackArgs pa{};
-    pa.W = gate->d_w;
-    pa.W2 = up->d_w;
-    pa.w_row0 = (int)f0;
-    pa.w_rows = (int)std::min(fc, ff - f0);
-    pa.K = c1.K;
-    pa.KS = KS1;
-    pa.KB = c1.KB;
-    pa.x = d_x;
-    pa.x_rows = f0 ? 0 : (int)rows;
-    pa.Wp = wp;
-    pa.Xp = xp;
-    pa.w_lo = 2 * fc * rb1 / planes;
-    pa.x_lo = xb / planes;
-    HIP_TRY(launch_pack(c1.type, pa, sp, s));
-    PackedGemmArgs a{};
-    a.Wp = wp;
-    a.Xp = xp;
-    a.w_bytes = (uint32_t)(2 * fc * rb1);
-    a.x_bytes = (uint32_t)xb;
-    a.w_lo = (uint32_t)pa.w_lo;
-    a.x_lo = (uint32_t)pa.x_lo;
-    a.m = 2 * pa.w_rows;
-    a.N = (int)rows;
-    a.KS = KS1;
-    a.splits = 1;
-    a.steps_per_split = c1.plan.steps_per_split;
-    a.Hp = hp + f0 / 16 * 1024;
-    a.h_lo = (uint32_t)(hb / planes);
-    a.KSh = KS2;
-    HIP_TRY(launch_packed_gemm(a, c1.plan.tile, sp, s));
-  }
-  float* partial = c2.plan.splits > 1 ? (float*)ws : nullptr;
-  for (size_t m0 = 0; m0 < d; m0 += dc) {
-    PackArgs pd{};
-    pd.W = down->d_w;
-    pd.w_row0 = (int)m0;
-    pd.w_rows = (int)std::min(dc, d - m0);
-    pd.K = c2.K;
-    pd.KS = KS2;
-    pd.KB = c2.KB;
-    pd.Wp = wp;
-    pd.w_lo = dc * rb2 / planes;
-    HIP_TRY(launch_pack(c2.type, pd, sp, s));
-    PackedGemmArgs b{};
-    b.Wp = wp;
-    b.Xp = hp;
-    b.w_bytes = (uint32_t)(dc * rb2);
-    b.x_bytes = (uint32_t)hb;
-    b.w_lo = (uint32_t)pd.w_lo;
-    b.x_lo = (uint32_t)(hb / planes);
-    b.Y = d_y + m0;
-    b.partial = partial ? partial + m0 : nullptr;
-    b.split_stride = rows * d;
-    b.m = pd.w_rows;
-    b.N = (int)rows;
-    b.KS = KS2;
-    b.ldy = c2.m;
-    b.splits = c2.plan.splits;
-    b.steps_per_split = c2.plan.steps_per_split;
-    b.add = partial || !d_add ? nullptr : d_add + m0;   // else in the reduce
-    HIP_TRY(launch_packed_gemm(b, c2.plan.tile, sp, s));
-  }
-  if (partial) HIP_TRY(launch_gemm_reduce(partial, d_y, rows * d, c2.plan.splits, s, d_add));
-  return RE_OK;
+  return with_packed_slot(total, s, ran, [&](void* buf, hipEvent_t done) -> int {
+    for (re_qmat* q : {gate, up, down}) warm_partials(q, rows, mode);
+    uint8_t* ws = (uint8_t*)buf;
+    uint8_t *xp = ws + part, *hp = xp + xb, *wp = hp + hb;
+    const int planes = sp ? 2 : 1, KS1 = (c1.K + 31) / 32 * 2, KS2 = (c2.K + 31) / 32 * 2;
+    for (size_t f0 = 0; f0 < ff; f0 += fc) {      // fc is a multiple of 128: whole slabs and h fragments
+      PackArgs pa{};
+      pa.W = gate->d_w;
+      pa.W2 = up->d_w;
+      pa.w_row0 = (int)f0;
+      pa.w_rows = (int)std::min(fc, ff - f0);
+      pa.K = c1.K;
+      pa.KS = KS1;
+      pa.KB = c1.KB;
+      pa.x = d_x;
+      pa.x_rows = f0 ? 0 : (int)rows;
+      pa.Wp = wp;
+      pa.Xp = xp;
+      pa.w_lo = 2 * fc * rb1 / planes;
+      pa.x_lo = xb / planes;
+      HIP_TRY(launch_pack(c1.type, pa, sp, s));
+      PackedGemmArgs a{};
+      a.Wp = wp;
+      a.Xp = xp;
+      a.w_bytes = (uint32_t)(2 * fc * rb1);
+      a.x_bytes = (uint32_t)xb;
+      a.w_lo = (uint32_t)pa.w_lo;
+      a.x_lo = (uint32_t)pa.x_lo;
+      a.m = 2 * pa.w_rows;
+      a.N = (int)rows;
+      a.KS = KS1;
+      a.splits = 1;
+      a.steps_per_split = c1.plan.steps_per_split;
+      a.Hp = hp + f0 / 16 * 1024;
+      a.h_lo = (uint32_t)(hb / planes);
+      a.KSh = KS2;
+      HIP_TRY(launch_packed_gemm(a, c1.plan.tile, sp, s));
+    }
+    float* partial = c2.plan.splits > 1 ? (float*)ws : nullptr;
+    for (size_t m0 = 0; m0 < d; m0 += dc) {
+      PackArgs pd{};
+      pd.W = down->d_w;
+      pd.w_row0 = (int)m0;
+      pd.w_rows = (int)std::min(dc, d - m0);
+      pd.K = c2.K;
+      pd.KS = KS2;
+      pd.KB = c2.KB;
+      pd.Wp = wp;
+      pd.w_lo = dc * rb2 / planes;
+      HIP_TRY(launch_pack(c2.type, pd, sp, s));
+      PackedGemmArgs b{};
+      b.Wp = wp;
+      b.Xp = hp;
+      b.w_bytes = (uint32_t)(dc * rb2);
+      b.x_bytes = (uint32_t)hb;
+      b.w_lo = (uint32_t)pd.w_lo;
+      b.x_lo = (uint32_t)(hb / planes);
+      b.Y = d_y + m0;
+      b.partial = partial ? partial + m0 : nullptr;
+      b.split_stride = rows * d;
+      b.m = pd.w_rows;
+      b.N = (int)rows;
+      b.KS = KS2;
+      b.ldy = c2.m;
+      b.splits = c2.plan.splits;
+      b.steps_per_split = c2.plan.steps_per_split;
+      b.add = partial || !d_add ? nullptr : d_add + m0;   // else in the reduce
+      HIP_TRY(launch_packed_gemm(b, c2.plan.tile, sp, s, !partial && m0 + dc >= d ? done : nullptr));
+    }
+    if (partial) HIP_TRY(launch_gemm_reduce(partial, d_y, rows * d, c2.plan.splits, s, d_add, done));
+    return RE_OK;
+  });
 }
 
 // fixed_partial: nullptr (the matrix's own partial buffer, grown on first use), or a caller-owned
@@ -1060,10 +1057,7 @@ int re_qmat_create(uint32_t ggml_type, const uint8_t* bytes, size_t nbytes, size
 
 void re_qmat_destroy(re_qmat* q) {
   if (!q) return;
-  if (q->stream) {
-    (void)hipStreamSynchronize(q->stream);
-    packed_idle(q->stream);
-  }
+  if (q->stream) (void)hipStreamSynchronize(q->stream);
   if (q->d_w) (void)hipFree(q->d_w);
   if (q->d_partial) (void)hipFree(q->d_partial);
   if (q->d_norm) (void)hipFree(q->d_norm);
@@ -1240,10 +1234,8 @@ namespace {
 constexpr int kScratchDevices = 64;
 std::mutex g_scratch_mu;
 float* g_scratch_dev[kScratchDevices] = {};
-// per device: an event recorded after the last no-allocation call's launches, and that call's
-// stream (a call on another stream waits on the event first)
+// per device: an event recorded after the last no-allocation call's launches (the next call waits for it)
 hipEvent_t g_scratch_ev[kScratchDevices] = {};
-hipStream_t g_scratch_last[kScratchDevices] = {};
 bool g_scratch_used[kScratchDevices] = {};
 
 // the calling thread's current device's copy of `scratch` and its ordering event, both set up
@@ -1287,13 +1279,13 @@ int re_qmat_matmul_noalloc_dev(re_qmat* q, const float* d_x, size_t rows, float*
   HIP_TRY(hipStreamIsCapturing(s, &cs));
   // under capture the caller orders the replays of graphs that share the scratch
   if (cs != hipStreamCaptureStatusNone) return enqueue(part, s);
-  // outside capture, calls on different streams of one GPU are ordered through the device's event
-  // (the lock also orders calls from different threads); calls on one stream are ordered by it
+  // outside capture, the calls on one GPU are ordered through the device's event whatever their streams
+  // (a new stream may have the handle of a destroyed one whose work is still in flight); the lock orders
+  // calls from different threads
   std::lock_guard<std::mutex> lk(g_scratch_mu);
-  if (g_scratch_used[dev] && g_scratch_last[dev] != s) HIP_TRY(hipStreamWaitEvent(s, g_scratch_ev[dev], 0));
+  if (g_scratch_used[dev]) HIP_TRY(hipStreamWaitEvent(s, g_scratch_ev[dev], 0));
   if ((rc = enqueue(part, s))) return rc;
   HIP_TRY(hipEventRecord(g_scratch_ev[dev], s));
-  g_scratch_last[dev] = s;
   g_scratch_used[dev] = true;
   return RE_OK;
 }
@@ -1321,7 +1313,6 @@ int re_qmat_matmul(re_qmat* q, const float* x, size_t rows, float* y, int mode) 
     if ((rc = re_qmat_matmul_dev(q, (const float*)q->sx.p, rows, (float*)q->sy.p, mode, q->stream))) return rc;
     HIP_TRY(hipMemcpyAsync(y, q->sy.p, yb, hipMemcpyDeviceToHost, q->stream));
     HIP_TRY(hipStreamSynchronize(q->stream));
-    packed_idle(q->stream);
     return RE_OK;
   }
   if ((rc = q->hx.ensure(xb)) || (rc = q->hy.ensure(yb))) return rc;
@@ -1332,7 +1323,6 @@ int re_qmat_matmul(re_qmat* q, const float* x, size_t rows, float* y, int mode) 
   if ((rc = re_qmat_matmul_dev(q, (const float*)q->sx.p, rows, dy, mode, q->stream))) return rc;
   if (io == 1) HIP_TRY(hipMemcpyAsync(q->hy.h, q->sy.p, yb, hipMemcpyDeviceToHost, q->stream));
   HIP_TRY(hipStreamSynchronize(q->stream));
-  packed_idle(q->stream);
   std::memcpy(y, q->hy.h, yb);
   return RE_OK;
 }

@@ -26,6 +26,7 @@
 //
 // Grouped launch (MoE): one task per workgroup names the expert, the weight tile and a run of
 // gathered activation rows; `xrow` maps a gathered row to its activation row.
+#include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -643,21 +644,22 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const V* __restrict__ 
 }
 
 static hipError_t launch_reduce(const float* partial, float* y, size_t n, int splits, hipStream_t s,
-                                const float* add = nullptr) {
-  if (n % 4 == 0 && ((uintptr_t)partial & 15) == 0 && ((uintptr_t)y & 15) == 0 && ((uintptr_t)add & 15) == 0) {
-    const size_t n4 = n / 4;
-    auto* k = add ? gemm_reduce_kernel<float4, true> : gemm_reduce_kernel<float4, false>;
-    hipLaunchKernelGGL(k, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s, (const float4*)partial, (float4*)y, n4,
-                       splits, (const float4*)add);
-  } else {
-    auto* k = add ? gemm_reduce_kernel<float, true> : gemm_reduce_kernel<float, false>;
-    hipLaunchKernelGGL(k, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, partial, y, n, splits, add);
-  }
-  return hipGetLastError();
+                                const float* add = nullptr, hipEvent_t done = nullptr) {
+  auto launch = [&](auto* k, size_t len, auto* p, auto* out, auto* a) {
+    const dim3 grid((unsigned)((len + 255) / 256));
+    if (done) hipExtLaunchKernelGGL(k, grid, dim3(256), 0, s, nullptr, done, 0, p, out, len, splits, a);
+    else hipLaunchKernelGGL(k, grid, dim3(256), 0, s, p, out, len, splits, a);
+    return hipGetLastError();
+  };
+  if (n % 4 == 0 && ((uintptr_t)partial & 15) == 0 && ((uintptr_t)y & 15) == 0 && ((uintptr_t)add & 15) == 0)
+    return launch(add ? gemm_reduce_kernel<float4, true> : gemm_reduce_kernel<float4, false>, n / 4,
+                  (const float4*)partial, (float4*)y, (const float4*)add);
+  return launch(add ? gemm_reduce_kernel<float, true> : gemm_reduce_kernel<float, false>, n, partial, y, add);
 }
 
-hipError_t launch_gemm_reduce(const float* partial, float* y, size_t n, int splits, hipStream_t s, const float* add) {
-  return launch_reduce(partial, y, n, splits, s, add);
+hipError_t launch_gemm_reduce(const float* partial, float* y, size_t n, int splits, hipStream_t s, const float* add,
+                              hipEvent_t done) {
+  return launch_reduce(partial, y, n, splits, s, add, done);
 }
 
 // x[i] -> bf16 with round to nearest even (the rounding the bf16-mode GEMM applies to f32 X), 8

@@ -200,7 +200,9 @@ struct PackedGemmArgs {
   uint32_t h_lo = 0;
   int KSh = 0;
 };
-hipError_t launch_packed_gemm(const PackedGemmArgs& a, PackedTile tile, bool sp, hipStream_t s);
+// done: an event that the launch's end completes (nullptr: none)
+hipError_t launch_packed_gemm(const PackedGemmArgs& a, PackedTile tile, bool sp, hipStream_t s,
+                              hipEvent_t done = nullptr);
 // Few-row dense GEMM (skinny.hip): Y[N x m] = X[N x K] W^T for N <= 64 rows of f32 X, a 64-row
 // weight tile and a K slice of blocks_per_split whole blocks per workgroup; splits > 1 writes
 // partial[split][N][ldy] for the split-K reduce (launch with launch_gemm_reduce).
@@ -223,10 +225,10 @@ SkinnyPlan plan_skinny(int m, int K, int qk);
 size_t skinny_lds_bytes(int staged_k, bool split_operands);
 // split_operands: f32 mode (split bf16 operands, three MFMAs per product)
 hipError_t launch_gemm_skinny(uint32_t type, const SkinnyArgs& a, bool split_operands, hipStream_t s);
-// y = sum over splits, in split order, of partial[split] (n floats each), streaming stores
-// y = (add +) the slices' sum; add may be y
+// y = (add +) the sum over splits, in split order, of partial[split] (n floats each), streaming stores;
+// add may be y; done: an event that the launch's end completes (nullptr: none)
 hipError_t launch_gemm_reduce(const float* partial, float* y, size_t n, int splits, hipStream_t s,
-                              const float* add = nullptr);
+                              const float* add = nullptr, hipEvent_t done = nullptr);
 
 // xb[i] = bf16(x[i]), round to nearest even; n a multiple of 8, both buffers 16-byte aligned
 hipError_t launch_x_to_bf16(const float* x, void* xb, size_t n, hipStream_t s);

@@ -16,6 +16,7 @@
 // f32 mode (SP): a second plane of each operand holds the bf16 rounding of what the first leaves,
 // and every product is w_hi x_hi + w_hi x_lo + w_lo x_hi in f32 accumulators, each term within
 // 2^-16 relative, as in the tiled GEMM.
+#include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -374,10 +375,12 @@ __global__ __launch_bounds__(WM* WN * 64) void packed_gemm_kernel(PackedGemmArgs
 }
 
 template <int BM, int BN, int WM, int WN, int KK, int NB, bool SP, bool SW = false>
-hipError_t launch_shape(const PackedGemmArgs& a, hipStream_t s) {
+hipError_t launch_shape(const PackedGemmArgs& a, hipStream_t s, hipEvent_t done) {
   const int total = ((a.m + BM - 1) / BM) * ((a.N + BN - 1) / BN) * a.splits;
   const int grid = (total + 7) / 8 * 8;
-  hipLaunchKernelGGL((packed_gemm_kernel<BM, BN, WM, WN, KK, NB, SP, SW>), dim3((unsigned)grid), dim3(WM * WN * 64), 0, s, a);
+  auto* k = packed_gemm_kernel<BM, BN, WM, WN, KK, NB, SP, SW>;
+  if (done) hipExtLaunchKernelGGL(k, dim3((unsigned)grid), dim3(WM * WN * 64), 0, s, nullptr, done, 0, a);
+  else hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(WM * WN * 64), 0, s, a);
   return hipGetLastError();
 }
 
@@ -414,36 +417,36 @@ hipError_t launch_pack(uint32_t type, PackArgs a, bool sp, hipStream_t s) {
   }
 }
 
-hipError_t launch_packed_gemm(const PackedGemmArgs& a, PackedTile tile, bool sp, hipStream_t s) {
+hipError_t launch_packed_gemm(const PackedGemmArgs& a, PackedTile tile, bool sp, hipStream_t s, hipEvent_t done) {
   if (a.Hp) {
     if (a.splits != 1) return hipErrorInvalidValue;
     if (sp) {
       switch (tile) {
-        case PackedTile::k256x128: return launch_shape<256, 128, 4, 2, 2, 3, true, true>(a, s);
-        case PackedTile::k128x128: return launch_shape<128, 128, 2, 2, 2, 4, true, true>(a, s);
-        case PackedTile::k128x64: return launch_shape<128, 64, 2, 2, 2, 3, true, true>(a, s);
+        case PackedTile::k256x128: return launch_shape<256, 128, 4, 2, 2, 3, true, true>(a, s, done);
+        case PackedTile::k128x128: return launch_shape<128, 128, 2, 2, 2, 4, true, true>(a, s, done);
+        case PackedTile::k128x64: return launch_shape<128, 64, 2, 2, 2, 3, true, true>(a, s, done);
         default: return hipErrorInvalidValue;
       }
     }
     switch (tile) {
-      case PackedTile::k256x256: return launch_shape<256, 256, 2, 4, 2, 4, false, true>(a, s);
-      case PackedTile::k128x128: return launch_shape<128, 128, 2, 2, 2, 4, false, true>(a, s);
+      case PackedTile::k256x256: return launch_shape<256, 256, 2, 4, 2, 4, false, true>(a, s, done);
+      case PackedTile::k128x128: return launch_shape<128, 128, 2, 2, 2, 4, false, true>(a, s, done);
       default: return hipErrorInvalidValue;
     }
   }
   if (sp) {
     switch (tile) {
-      case PackedTile::k256x128: return launch_shape<256, 128, 4, 2, 2, 3, true>(a, s);
-      case PackedTile::k192x128: return launch_shape<192, 128, 2, 2, 2, 4, true>(a, s);
-      case PackedTile::k128x128: return launch_shape<128, 128, 2, 2, 2, 4, true>(a, s);
-      case PackedTile::k128x64: return launch_shape<128, 64, 2, 2, 2, 3, true>(a, s);
+      case PackedTile::k256x128: return launch_shape<256, 128, 4, 2, 2, 3, true>(a, s, done);
+      case PackedTile::k192x128: return launch_shape<192, 128, 2, 2, 2, 4, true>(a, s, done);
+      case PackedTile::k128x128: return launch_shape<128, 128, 2, 2, 2, 4, true>(a, s, done);
+      case PackedTile::k128x64: return launch_shape<128, 64, 2, 2, 2, 3, true>(a, s, done);
       default: return hipErrorInvalidValue;
     }
   }
   switch (tile) {
-    case PackedTile::k256x256: return launch_shape<256, 256, 2, 4, 2, 4, false>(a, s);
-    case PackedTile::k192x128: return launch_shape<192, 128, 2, 2, 2, 4, false>(a, s);
-    case PackedTile::k128x128: return launch_shape<128, 128, 2, 2, 2, 4, false>(a, s);
+    case PackedTile::k256x256: return launch_shape<256, 256, 2, 4, 2, 4, false>(a, s, done);
+    case PackedTile::k192x128: return launch_shape<192, 128, 2, 2, 2, 4, false>(a, s, done);
+    case PackedTile::k128x128: return launch_shape<128, 128, 2, 2, 2, 4, false>(a, s, done);
     default: return hipErrorInvalidValue;
   }
 }

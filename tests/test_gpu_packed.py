@@ -134,6 +134,35 @@ def test_streams_and_capture():
         q.close()
 
 
+def test_streams_come_and_go():
+    """Streams made, used and destroyed while their work may still run, more of them than workspaces, and
+    new ones (which may get old handles) in their place: every call gets the bits of the first."""
+    m, n, rows = 896, 4864, 400
+    rng = np.random.default_rng(7)
+    q = rehip.QMat.from_bytes(rehip.Q6_K, weights(rng, rehip.Q6_K, m, n), m, n)
+    big = rehip.QMat.from_bytes(rehip.Q4_0, weights(rng, rehip.Q4_0, 4096, 4096), 4096, 4096)
+    dx, dxb = B.from_array(synth.activations(rng, rows, n)), B.from_array(synth.activations(rng, rows, 4096))
+    want, yb = run(q, dx, rows, m, rehip.MODE_F32), B(rows * 4096 * 4)
+    for turn in range(4):
+        streams = [hip.Stream() for _ in range(6 + turn)]
+        ys = [B(rows * m * 4) for _ in streams]
+        for s, y in zip(streams, ys):
+            if turn == 2:
+                big.matmul_dev(dxb, rows, yb, rehip.MODE_F32, stream=s)      # a larger workspace on the way
+            q.matmul_dev(dx, rows, y, rehip.MODE_F32, stream=s)
+        for s in streams:
+            s.destroy()
+        again = hip.Stream()
+        y2 = B(rows * m * 4)
+        q.matmul_dev(dx, rows, y2, rehip.MODE_F32, stream=again)
+        hip.synchronize()
+        for y in ys + [y2]:
+            assert np.array_equal(y.download(np.float32, rows * m), want)
+        again.destroy()
+    q.close()
+    big.close()
+
+
 def test_capture_after_eager_call_keeps_its_slices():
     """A graph captured after an eager call (which ran on packed operands) takes the tiled GEMM with its
     K slices: the bits of a call that never packs."""
