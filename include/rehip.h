@@ -104,8 +104,9 @@ int re_qmat_matmul_dev(re_qmat *q, const float *d_x, size_t rows, float *d_y, in
  * every shape fit: the planner caps partial tiles at 32 MiB). The scratch
  * is shared by every call on a GPU. Outside stream capture, a call first waits for the launches of the
  * previous call on that GPU (an event set up once per device), so calls from several streams or threads
- * stay ordered. Inside stream capture no
- * ordering is added: replays of captured graphs that use the scratch must not overlap in time. */
+ * stay ordered. Inside stream capture no ordering is added: replays of captured graphs that use the
+ * scratch must not overlap in time. Those are the graphs of quantized calls with K slices; dense weights
+ * and single-slice calls are captured without the scratch, as the unpacked GEMM. */
 int re_qmat_matmul_noalloc_dev(re_qmat *q, const float *d_x, size_t rows, float *d_y, int mode, void *stream);
 /* Dequantize the resident weights to d_out[m x n] f32, bit-exact with quant::dequant. */
 int re_qmat_dequant_dev(re_qmat *q, float *d_out, void *stream);

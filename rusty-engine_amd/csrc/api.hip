@@ -875,16 +875,24 @@ int gemm_enqueue(re_qmat* q, const float* d_x, size_t rows, float* d_y, int mode
       return RE_OK;
     }
   }
-  PackedCall pc;
-  if (packed_call(q->g.type, q->d_w, q->g.m, q->g.n, q->g.kb, d_x, rows, mode, &pc)) {
-    if (fixed_partial) return packed_enqueue(pc, d_x, d_y, fixed_partial, fixed_cap, s);
-    bool ran = false;
-    const int rc = packed_shared(q, pc, d_x, d_y, mode, s, &ran);
-    if (rc || ran) return rc;
-  }
   // f32 mode on bf16 MFMAs with split operands (REHIP_GEMM_SP=0: the f32 MFMA tiles)
   const int kmode = mode == RE_MODE_F32 && env_size("REHIP_GEMM_SP", 1) != 0 ? kGemmModeSplit : mode;
   GemmPlan pl = plan_gemm((int)q->g.m, (int)rows, (int)q->g.n, kmode);
+  PackedCall pc;
+  if (packed_call(q->g.type, q->d_w, q->g.m, q->g.n, q->g.kb, d_x, rows, mode, &pc)) {
+    if (fixed_partial) {
+      // captured: packed operands only where the tiled GEMM's K slices would be in the scratch too, so that
+      // the graphs of the other calls need no ordering among each other
+      hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+      HIP_TRY(hipStreamIsCapturing(s, &cs));
+      if (cs == hipStreamCaptureStatusNone || pl.splits > 1)
+        return packed_enqueue(pc, d_x, d_y, fixed_partial, fixed_cap, s);
+    } else {
+      bool ran = false;
+      const int rc = packed_shared(q, pc, d_x, d_y, mode, s, &ran);
+      if (rc || ran) return rc;
+    }
+  }
   // tuning knobs: REHIP_GEMM_TILE (1 64x64, 2 128x128, 3 128x256, 4 256x128, 5 128x192), REHIP_GEMM_KG,
   // REHIP_GEMM_SPLITS; a combination the library does not build fails at launch
   if (const size_t t = env_size("REHIP_GEMM_TILE", 0); t >= 1 && t <= 5) {
@@ -1262,8 +1270,12 @@ int re_qmat_matmul_noalloc_dev(re_qmat* q, const float* d_x, size_t rows, float*
   if (!q || (rows && (!d_x || !d_y))) return fail(RE_ERR_ARG, "null pointer");
   if (mode != RE_MODE_BF16 && mode != RE_MODE_F32) return fail(RE_ERR_ARG, "unknown mode %d", mode);
   if (rows == 0) return RE_OK;
+  const hipStream_t s = (hipStream_t)stream;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  HIP_TRY(hipStreamIsCapturing(s, &cs));
+  const bool capturing = cs != hipStreamCaptureStatusNone;
   PackedCall pc;
-  const bool packed = q->dense && dense_packed(q, d_x, rows, mode, &pc);
+  const bool packed = q->dense && !capturing && dense_packed(q, d_x, rows, mode, &pc);
   if (rows == 1 || (q->dense && !packed)) return re_qmat_matmul_dev(q, d_x, rows, d_y, mode, stream);   // no scratch
   if (rows > (1u << 24)) return fail(RE_ERR_SIZE, "rows = %zu too large", rows);
   auto enqueue = [&](float* scratch_dev, hipStream_t st) {
@@ -1274,11 +1286,8 @@ int re_qmat_matmul_noalloc_dev(re_qmat* q, const float* d_x, size_t rows, float*
   int dev = 0;
   int rc = scratch_for_current_device(&part, &dev);
   if (rc) return rc;
-  const hipStream_t s = (hipStream_t)stream;
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  HIP_TRY(hipStreamIsCapturing(s, &cs));
   // under capture the caller orders the replays of graphs that share the scratch
-  if (cs != hipStreamCaptureStatusNone) return enqueue(part, s);
+  if (capturing) return enqueue(part, s);
   // outside capture, the calls on one GPU are ordered through the device's event whatever their streams
   // (a new stream may have the handle of a destroyed one whose work is still in flight); the lock orders
   // calls from different threads

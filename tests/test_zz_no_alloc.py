@@ -124,3 +124,37 @@ def test_noalloc_two_streams_without_host_sync():
     sb.destroy()
     qa.close()
     qb.close()
+
+
+@pytest.mark.parametrize("t,m,n,rows", [(rehip.Q5_K, 4864, 1024, 512), (rehip.F16, 4864, 896, 512)])
+def test_captured_calls_of_one_slice_use_no_scratch(t, m, n, rows):
+    # single-slice and dense calls are captured without the scratch: two graphs of them replayed side by
+    # side, with an eager call on packed operands between them, each get the unpacked GEMM's bits
+    rng = np.random.default_rng(8100 + t)
+    qs, dx, want = [], [], []
+    for _ in range(2):
+        w = (rng.standard_normal((m, n)).astype(np.float16).view(np.uint8).reshape(-1) if t == rehip.F16
+             else synth.weight_bytes(rng, t, m, n))
+        qs.append(rehip.QMat.from_bytes(t, w, m, n))
+        dx.append(hip.DeviceBuffer.from_array(synth.activations(rng, rows, n)))
+    ys = [hip.DeviceBuffer(rows * m * 4) for _ in range(3)]
+    with pytest.MonkeyPatch.context() as mp:
+        mp.setenv("REHIP_GEMM_PACKED", "0")
+        for q, x in zip(qs, dx):
+            q.matmul_dev(x, rows, ys[0], rehip.MODE_F32)
+            hip.synchronize()
+            want.append(ys[0].download(np.float32, rows * m))
+    ss = [hip.Stream() for _ in range(3)]
+    gs = [hip.Graph(s, lambda q=q, x=x, y=y, s=s: q.matmul_noalloc_dev(x, rows, y, rehip.MODE_F32, stream=s))
+          for q, x, y, s in zip(qs, dx, ys, ss)]
+    for rep in range(4):
+        for g in gs:
+            g.launch()
+        qs[0].matmul_noalloc_dev(dx[0], rows, ys[2], rehip.MODE_F32, stream=ss[2])
+        hip.synchronize()
+        for y, v in zip(ys, want):
+            assert np.array_equal(y.download(np.float32, rows * m), v), rep
+    for o in gs + ss:
+        o.destroy()
+    for q in qs:
+        q.close()
