@@ -673,26 +673,37 @@ int packed_enqueue(const PackedCall& c, const float* d_x, float* d_y, void* ws, 
   return RE_OK;
 }
 
+// The few-row GEMM (skinny.hip) serves 2..32 rows in bf16 mode (one 32-row token tile) and 2..64 rows in
+// f32 mode, where the tiled GEMM stages f32 tiles; it is faster than the tiled GEMM there. REHIP_SKINNY=0
+// keeps the tiled GEMM for A/B runs.
+bool few_rows(const float* d_x, size_t rows, int mode) {
+  return rows >= 2 && rows <= (mode == RE_MODE_F32 ? 64u : 32u) && aligned16(d_x) &&
+         env_size("REHIP_SKINNY", 1) != 0 && !env_size("REHIP_GEMM_TILE", 0);
+}
+
 // Grow the matrix's K-split partials for the GEMM that a captured call of this shape takes, as an eager
 // call of it would (a graph captured after an eager call on packed operands otherwise ran unsplit: Q6_K
 // 896 x 4864, 961 rows, 106 instead of 29 us). Out of memory only costs the split.
-void warm_partials(re_qmat* q, size_t rows, int mode) {
+void warm_partials(re_qmat* q, const float* d_x, size_t rows, int mode) {
   int splits = 1;
   if (q->dense) {
     splits = dense_mma_splits((int)q->g.m, (int)q->g.n, (int)rows);
     if ((size_t)splits * rows * q->g.m * sizeof(float) > (32u << 20)) return;
+  } else if (few_rows(d_x, rows, mode)) {
+    splits = plan_skinny((int)q->g.m, (int)q->g.n, (int)q->g.qk).splits;
   } else {
     splits = plan_gemm((int)q->g.m, (int)rows, (int)q->g.n, mode == RE_MODE_F32 ? kGemmModeSplit : mode).splits;
   }
   const size_t need = (size_t)splits * rows * q->g.m * sizeof(float);
-  if (splits > 1 && need > q->spart.cap) (void)q->spart.ensure(need);
+  if (splits > 1 && need > q->spart.cap && q->spart.ensure(need) != RE_OK)
+    (void)hipGetLastError();                      // else the next launch would return it
 }
 
 // The call on packed operands, in a workspace of the GPU's (*ran as in with_packed_slot).
 int packed_shared(re_qmat* q, const PackedCall& c, const float* d_x, float* d_y, int mode, hipStream_t s, bool* ran) {
   const size_t bytes = c.want(kPackedWsBytes);
   return with_packed_slot(bytes, s, ran, [&](void* ws, hipEvent_t done) {
-    warm_partials(q, c.rows, mode);
+    warm_partials(q, d_x, c.rows, mode);
     return packed_enqueue(c, d_x, d_y, ws, bytes, s, done);
   });
 }
@@ -743,7 +754,7 @@ int packed_ffn(re_qmat* gate, re_qmat* up, re_qmat* down, const float* d_x, size
   if (fc == 0 || dc == 0) return RE_OK;
   const size_t total = fixed + region;
   return with_packed_slot(total, s, ran, [&](void* buf, hipEvent_t done) -> int {
-    for (re_qmat* q : {gate, up, down}) warm_partials(q, rows, mode);
+    for (re_qmat* q : {gate, up, down}) warm_partials(q, d_x, rows, mode);
     uint8_t* ws = (uint8_t*)buf;
     uint8_t *xp = ws + part, *hp = xp + xb, *wp = hp + hb;
     const int planes = sp ? 2 : 1, KS1 = (c1.K + 31) / 32 * 2, KS2 = (c2.K + 31) / 32 * 2;
@@ -823,13 +834,9 @@ int gemm_enqueue(re_qmat* q, const float* d_x, size_t rows, float* d_y, int mode
   const size_t xbytes = rows * q->g.n * sizeof(float);
   if (xbytes >= (1ull << 31) || q->g.bytes >= (1ull << 31))
     return fail(RE_ERR_SIZE, "GEMM operands must stay below 2 GiB (X %zu B, W %zu B)", xbytes, q->g.bytes);
-  // few rows: the few-row GEMM (weights decoded in registers, one workgroup per 64-row tile and
-  // K slice, K slices for ~256 workgroups). It is faster than the tiled GEMM for 2..32 rows in bf16
-  // mode (one 32-row token tile) and for 2..64 rows in f32 mode, where the tiled GEMM stages f32
-  // tiles. REHIP_SKINNY=0 keeps the tiled GEMM for A/B runs.
-  const size_t skinny_max = mode == RE_MODE_F32 ? 64 : 32;
-  if (rows >= 2 && rows <= skinny_max && aligned16(d_x) && env_size("REHIP_SKINNY", 1) != 0 &&
-      !env_size("REHIP_GEMM_TILE", 0)) {
+  // few rows: weights decoded in registers, one workgroup per 64-row tile and K slice, K slices for ~256
+  // workgroups
+  if (few_rows(d_x, rows, mode)) {
     const SkinnyPlan sp = plan_skinny((int)q->g.m, (int)q->g.n, (int)q->g.qk);
     SkinnyArgs a{};
     a.W = q->d_w;

@@ -116,6 +116,40 @@ def test_one_matrix_as_gate_and_up(mode):
         m.close()
 
 
+def test_capture_after_eager_call_keeps_its_slices():
+    """A captured FFN (separate calls) after an eager one on packed operands, at the row count that the
+    few-row GEMM serves: its K slices, so the bits of separate calls that never packed."""
+    d, ff, rows = 896, 4864, 64
+    rng = np.random.default_rng(12)
+    w = matrices(rng, rehip.Q4_K, rehip.Q6_K, d, ff)
+    x = B.from_array((0.1 * synth.activations(rng, rows, d)).astype(np.float32))
+    got = []
+    for packed in (True, False):
+        q = [rehip.QMat.from_bytes(t, b, *s) for t, b, s in zip((rehip.Q4_K, rehip.Q4_K, rehip.Q6_K), w,
+                                                                ((ff, d), (ff, d), (d, ff)))]
+        f = rehip.Ffn(q[0], q[1])
+        wb = f.block_work_bytes(q[2], rows)
+        y, wk, s = B(rows * d * 4), B(wb), hip.Stream()
+
+        def call():
+            f.block_dev(q[2], x, rows, y, wk, wb, rehip.MODE_F32, stream=s)
+        with pytest.MonkeyPatch.context() as mp:
+            if not packed:
+                mp.setenv("REHIP_GEMM_PACKED", "0")
+            call()
+            g = hip.Graph(s, call)
+        for _ in range(3):
+            g.launch()
+            hip.synchronize()
+        got.append(y.download(np.float32, rows * d))
+        g.destroy()
+        s.destroy()
+        f.close()
+        for m in q:
+            m.close()
+    assert np.array_equal(got[0], got[1])
+
+
 def test_errors():
     rng = np.random.default_rng(1)
     w = matrices(rng, rehip.Q4_0, rehip.Q4_0, 64, 96)
