@@ -99,10 +99,11 @@ int re_qmat_matmul_dev(re_qmat *q, const float *d_x, size_t rows, float *d_y, in
  * (code under HIP graph capture, serving loops, harnesses that forbid hipMalloc). It has no
  * counterpart in the reference. The GEMM's K-split partial tiles and packed operands go to a static
  * device scratch of 64 MiB per GPU instead of buffers allocated on first use; the same plan, kernels
- * and results as re_qmat_matmul_dev (operands larger than the scratch are packed and multiplied in
- * pieces). A plan whose partials exceed the scratch fails with RE_ERR_SIZE (the planned splits of
- * every shape fit: the planner caps partial tiles at 32 MiB). The scratch
- * is shared by every call on a GPU. Outside stream capture, a call first waits for the launches of the
+ * and results as re_qmat_matmul_dev, except where packed operands exceed the scratch: they are then packed
+ * and multiplied in pieces (the same results) or, if the pieces would be too small to fill the GPU, the
+ * unpacked GEMM runs (results that differ by the order of the sums). A plan whose partials exceed the
+ * scratch fails with RE_ERR_SIZE (the planned splits of every shape fit: the planner caps partial tiles at
+ * 32 MiB). The scratch is shared by every call on a GPU. Outside stream capture, a call first waits for the launches of the
  * previous call on that GPU (an event set up once per device), so calls from several streams or threads
  * stay ordered. Inside stream capture no ordering is added: replays of captured graphs that use the
  * scratch must not overlap in time. Those are the graphs of quantized calls with K slices; dense weights

@@ -587,9 +587,9 @@ bool packed_pays(bool dense, size_t m, size_t K, size_t rows, bool sp) {
   return rows >= 384 || (rows >= 192 && K >= 1024 && (double)m * K * rows >= 3e9);
 }
 
-// Whether a call runs on packed operands, from its shape, type, mode and alignment alone (so that both
-// GEMM entry points take the same kernels). Rows longer than the no-allocation entry point's scratch
-// can hold stay with the tiled GEMM. REHIP_GEMM_PACKED: 0 never, 2 wherever the kernels can.
+// Whether a call can and should run on packed operands, from its shape, type, mode and alignment alone, so
+// that both GEMM entry points take the same kernels where the operands fit (else see pieces_pay). Rows
+// longer than the no-allocation entry point's scratch can hold stay with the tiled GEMM. REHIP_GEMM_PACKED: 0 never, 2 wherever the kernels can.
 bool packed_call(uint32_t type, const void* W, size_t m, size_t K, size_t KB, const float* d_x, size_t rows, int mode,
                  PackedCall* c) {
   const bool sp = mode == RE_MODE_F32;
@@ -616,17 +616,51 @@ bool dense_packed(const re_qmat* q, const float* d_x, size_t rows, int mode, Pac
          packed_call(q->g.type, q->d_w, q->g.m, q->g.n, 0, d_x, rows, mode, c);
 }
 
+// Rows of each operand packed at a time in a workspace of ws_bytes (whole operands if they fit); false: too
+// small for any.
+bool packed_pieces(const PackedCall& c, size_t ws_bytes, size_t* mc, size_t* nc) {
+  const size_t rb = c.row_bytes(), part = c.partial_bytes();
+  *mc = PackedCall::pad(c.m);
+  *nc = PackedCall::pad(c.rows);
+  if (part >= ws_bytes) return false;
+  const size_t most = (ws_bytes - part) / rb;
+  if (*mc + *nc <= most) return true;
+  *nc = std::min(*nc, std::max<size_t>(kPackedRows, most / 2 / kPackedRows * kPackedRows));
+  if (*nc >= most) return false;
+  *mc = std::min(*mc, (most - *nc) / kPackedRows * kPackedRows);
+  return *mc > 0;
+}
+
+// Whether a call whose operands do not fit the workspace whole is worth its pieces: they run one after
+// the other, so each has to fill the CUs. Measured in the static scratch of 64 MiB over m, K 896 .. 28672 and
+// 256 .. 4096 rows, against the ratio of the pieces' estimates (and 5 us for each further piece's launches
+// and drained end) to that of the whole product. Quantized weights win up to 1.4 from 768 rows (Q4_K, us
+// tiled / pieces: m x K 14336 x 4096, 2048 rows, bf16 349 / 256, f32 1178 / 646; 8192 x 8192, 2048 rows, bf16 374 /
+// 314) and lose from 1.55 or below (8192 x 8192, 1024 rows, bf16 186 / 198; 2048 x 8192, 512 rows, f32 75 / 83; 4096 x
+// 14336, 2048 rows, f32, 32 pieces: 1177 / 4467). Dense weights, whose tiled GEMM is slower, win up to 2
+// at any rows (F16 14336 x 4096, 512 rows, bf16 217 / 120) and lose from 2.1 (8192 x 2048, 256 rows, f32 61 / 76).
+bool pieces_pay(const PackedCall& c, size_t ws_bytes) {
+  size_t mc, nc;
+  if (!packed_pieces(c, ws_bytes, &mc, &nc)) return false;
+  if (mc >= (size_t)c.m && nc >= (size_t)c.rows) return true;
+  if (env_size("REHIP_GEMM_PACKED", 1) == 2) return true;
+  const bool dense = dense_type(c.type);
+  if (!dense && c.rows < 768) return false;
+  double us = 0;
+  int pieces = 0;
+  for (size_t n0 = 0; n0 < (size_t)c.rows; n0 += nc)
+    for (size_t m0 = 0; m0 < (size_t)c.m; m0 += mc, ++pieces)
+      us += plan_packed((int)std::min(mc, c.m - m0), (int)std::min(nc, c.rows - n0), c.K, c.sp, false, c.plan.splits).us;
+  return us + 5.0 * (pieces - 1) <= (dense ? 2.0 : 1.4) * c.plan.us;
+}
+
 // done: carried by the last launch (nullptr: none)
 int packed_enqueue(const PackedCall& c, const float* d_x, float* d_y, void* ws, size_t ws_bytes, hipStream_t s,
                    hipEvent_t done = nullptr) {
-  const size_t rb = c.row_bytes(), part = c.partial_bytes(), avail = ws_bytes - part;
-  const size_t mp = PackedCall::pad(c.m), np = PackedCall::pad(c.rows);
-  size_t mc = mp, nc = np;                       // rows of each operand packed at a time
-  if ((mp + np) * rb > avail) {
-    nc = std::min(np, std::max<size_t>(kPackedRows, avail / 2 / rb / kPackedRows * kPackedRows));
-    mc = std::min(mp, (avail - nc * rb) / rb / kPackedRows * kPackedRows);
-    if (mc == 0) return fail(RE_ERR_SIZE, "packed GEMM workspace of %zu bytes is too small", ws_bytes);
-  }
+  const size_t rb = c.row_bytes(), part = c.partial_bytes(), mp = PackedCall::pad(c.m);
+  size_t mc, nc;
+  if (!packed_pieces(c, ws_bytes, &mc, &nc))
+    return fail(RE_ERR_SIZE, "packed GEMM workspace of %zu bytes is too small", ws_bytes);
   const int KS = (c.K + 31) / 32 * 2, planes = c.sp ? 2 : 1;
   float* partial = c.plan.splits > 1 ? (float*)ws : nullptr;
   uint8_t* wp = (uint8_t*)ws + part;
@@ -665,8 +699,12 @@ int packed_enqueue(const PackedCall& c, const float* d_x, float* d_y, void* ws, 
       a.ldy = c.m;
       a.splits = c.plan.splits;
       a.steps_per_split = c.plan.steps_per_split;
+      // a piece's own tile, the whole product's K slices: the same sums
+      const PackedTile tile = mr == (size_t)c.m && rows == (size_t)c.rows
+                                  ? c.plan.tile
+                                  : plan_packed((int)mr, (int)rows, c.K, c.sp, false, c.plan.splits).tile;
       const bool last = n0 + nc >= (size_t)c.rows && m0 + mc >= (size_t)c.m;
-      HIP_TRY(launch_packed_gemm(a, c.plan.tile, c.sp, s, last && !partial ? done : nullptr));
+      HIP_TRY(launch_packed_gemm(a, tile, c.sp, s, last && !partial ? done : nullptr));
     }
   }
   if (partial) HIP_TRY(launch_gemm_reduce(partial, d_y, (size_t)c.rows * c.m, c.plan.splits, s, nullptr, done));
@@ -702,6 +740,8 @@ void warm_partials(re_qmat* q, const float* d_x, size_t rows, int mode) {
 // The call on packed operands, in a workspace of the GPU's (*ran as in with_packed_slot).
 int packed_shared(re_qmat* q, const PackedCall& c, const float* d_x, float* d_y, int mode, hipStream_t s, bool* ran) {
   const size_t bytes = c.want(kPackedWsBytes);
+  *ran = false;
+  if (!pieces_pay(c, bytes)) return RE_OK;
   return with_packed_slot(bytes, s, ran, [&](void* ws, hipEvent_t done) {
     warm_partials(q, d_x, c.rows, mode);
     return packed_enqueue(c, d_x, d_y, ws, bytes, s, done);
@@ -892,7 +932,7 @@ int gemm_enqueue(re_qmat* q, const float* d_x, size_t rows, float* d_y, int mode
       // the graphs of the other calls need no ordering among each other
       hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
       HIP_TRY(hipStreamIsCapturing(s, &cs));
-      if (cs == hipStreamCaptureStatusNone || pl.splits > 1)
+      if ((cs == hipStreamCaptureStatusNone || pl.splits > 1) && pieces_pay(pc, fixed_cap))
         return packed_enqueue(pc, d_x, d_y, fixed_partial, fixed_cap, s);
     } else {
       bool ran = false;
@@ -951,6 +991,36 @@ int gemm_enqueue(re_qmat* q, const float* d_x, size_t rows, float* d_y, int mode
     }
   }
   HIP_TRY(launch_gemm(q->g.type, kmode, a, 0, pl.tile, pl.kgroups, s));
+  return RE_OK;
+}
+
+// Dense weights: below 16 rows f32 products in either mode (the reference's f32 matvec); from 16 rows the
+// MFMA GEMM, bf16 operands in bf16 mode and split operands on bf16 MFMAs in f32 mode (REHIP_GEMM_SP=0: f32
+// MFMAs). pack: packed operands in a shared workspace may take it.
+int dense_enqueue(re_qmat* q, const float* d_x, size_t rows, float* d_y, int mode, hipStream_t s, bool pack) {
+  if (rows > 65535u * 4u) return fail(RE_ERR_SIZE, "rows = %zu too large for dense weights", rows);
+  PackedCall pc;
+  if (pack && dense_packed(q, d_x, rows, mode, &pc)) {
+    bool ran = false;
+    const int rc = packed_shared(q, pc, d_x, d_y, mode, s, &ran);
+    if (rc || ran) return rc;
+  }
+  int splits = 1;
+  if (dense_mma_rows((int)q->g.n, (int)rows, d_x)) {
+    // few output tiles: K slices into the matrix's partial buffer, grown on first use (under
+    // stream capture an unwarmed shape runs as one slice: the same result up to summation order)
+    splits = dense_mma_splits((int)q->g.m, (int)q->g.n, (int)rows);
+    const size_t need = (size_t)splits * rows * q->g.m * sizeof(float);
+    if (splits > 1 && need > q->spart.cap) {
+      hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+      HIP_TRY(hipStreamIsCapturing(s, &cs));
+      if (cs != hipStreamCaptureStatusNone || need > (32u << 20)) splits = 1;
+      else if (int rc = q->spart.ensure(need)) return rc;
+    }
+  }
+  const int kmode = mode == RE_MODE_F32 && env_size("REHIP_GEMM_SP", 1) != 0 ? kGemmModeSplit : mode;
+  HIP_TRY(launch_dense_gemm(q->g.type, q->d_w, d_x, d_y, (int)q->g.m, (int)q->g.n, (int)rows, nullptr, kmode,
+                            nullptr, splits > 1 ? (float*)q->spart.p : nullptr, splits, s));
   return RE_OK;
 }
 
@@ -1212,35 +1282,7 @@ int re_qmat_matmul_dev(re_qmat* q, const float* d_x, size_t rows, float* d_y, in
   if (mode != RE_MODE_BF16 && mode != RE_MODE_F32) return fail(RE_ERR_ARG, "unknown mode %d", mode);
   if (rows == 0) return RE_OK;
   if (rows > (1u << 24)) return fail(RE_ERR_SIZE, "rows = %zu too large", rows);
-  if (q->dense) {                        // below 16 rows f32 products in either mode (the reference's
-    // f32 matvec); from 16 rows the MFMA GEMM, bf16 operands in bf16 mode and split operands on
-    // bf16 MFMAs in f32 mode (REHIP_GEMM_SP=0: f32 MFMAs)
-    if (rows > 65535u * 4u) return fail(RE_ERR_SIZE, "rows = %zu too large for dense weights", rows);
-    const hipStream_t s = (hipStream_t)stream;
-    PackedCall pc;
-    if (dense_packed(q, d_x, rows, mode, &pc)) {
-      bool ran = false;
-      const int rc = packed_shared(q, pc, d_x, d_y, mode, s, &ran);
-      if (rc || ran) return rc;
-    }
-    int splits = 1;
-    if (dense_mma_rows((int)q->g.n, (int)rows, d_x)) {
-      // few output tiles: K slices into the matrix's partial buffer, grown on first use (under
-      // stream capture an unwarmed shape runs as one slice: the same result up to summation order)
-      splits = dense_mma_splits((int)q->g.m, (int)q->g.n, (int)rows);
-      const size_t need = (size_t)splits * rows * q->g.m * sizeof(float);
-      if (splits > 1 && need > q->spart.cap) {
-        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        HIP_TRY(hipStreamIsCapturing(s, &cs));
-        if (cs != hipStreamCaptureStatusNone || need > (32u << 20)) splits = 1;
-        else if (int rc = q->spart.ensure(need)) return rc;
-      }
-    }
-    const int kmode = mode == RE_MODE_F32 && env_size("REHIP_GEMM_SP", 1) != 0 ? kGemmModeSplit : mode;
-    HIP_TRY(launch_dense_gemm(q->g.type, q->d_w, d_x, d_y, (int)q->g.m, (int)q->g.n, (int)rows, nullptr, kmode,
-                              nullptr, splits > 1 ? (float*)q->spart.p : nullptr, splits, s));
-    return RE_OK;
-  }
+  if (q->dense) return dense_enqueue(q, d_x, rows, d_y, mode, (hipStream_t)stream, true);
   if (rows == 1) return gemv_enqueue(q, d_x, d_y, (hipStream_t)stream);
   return gemm_enqueue(q, d_x, rows, d_y, mode, (hipStream_t)stream);
 }
@@ -1281,10 +1323,11 @@ int re_qmat_matmul_noalloc_dev(re_qmat* q, const float* d_x, size_t rows, float*
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   HIP_TRY(hipStreamIsCapturing(s, &cs));
   const bool capturing = cs != hipStreamCaptureStatusNone;
-  PackedCall pc;
-  const bool packed = q->dense && !capturing && dense_packed(q, d_x, rows, mode, &pc);
-  if (rows == 1 || (q->dense && !packed)) return re_qmat_matmul_dev(q, d_x, rows, d_y, mode, stream);   // no scratch
+  if (rows == 1 && !q->dense) return gemv_enqueue(q, d_x, d_y, s);   // no scratch
   if (rows > (1u << 24)) return fail(RE_ERR_SIZE, "rows = %zu too large", rows);
+  PackedCall pc;
+  const bool packed = q->dense && !capturing && dense_packed(q, d_x, rows, mode, &pc) && pieces_pay(pc, kScratchBytes);
+  if (q->dense && !packed) return dense_enqueue(q, d_x, rows, d_y, mode, s, false);   // no scratch
   auto enqueue = [&](float* scratch_dev, hipStream_t st) {
     return packed ? packed_enqueue(pc, d_x, d_y, scratch_dev, kScratchBytes, st)
                   : gemm_enqueue(q, d_x, rows, d_y, mode, st, scratch_dev, kScratchBytes);

@@ -181,9 +181,11 @@ enum class PackedTile { k256x256, k256x128, k192x128, k128x128, k128x64 };   // 
 struct PackedPlan {
   PackedTile tile = PackedTile::k128x128;
   int splits = 1, steps_per_split = 1;
+  double us = 0;           // the estimate it was chosen by
 };
-// pairs: the SwiGLU epilogue (one K slice, whole gate / up pairs per wave)
-PackedPlan plan_packed(int m, int rows, int K, bool sp, bool pairs = false);
+// pairs: the SwiGLU epilogue (one K slice, whole gate / up pairs per wave); splits: the K slices of a
+// piece of a larger product (0: free)
+PackedPlan plan_packed(int m, int rows, int K, bool sp, bool pairs = false, int splits = 0);
 struct PackedGemmArgs {
   const uint8_t *Wp, *Xp;
   uint32_t w_bytes, x_bytes;   // all planes

@@ -451,7 +451,7 @@ hipError_t launch_packed_gemm(const PackedGemmArgs& a, PackedTile tile, bool sp,
   }
 }
 
-PackedPlan plan_packed(int m, int rows, int K, bool sp, bool pairs) {
+PackedPlan plan_packed(int m, int rows, int K, bool sp, bool pairs, int splits) {
   // The fullest CU's tiles times the stages of one, at the measured time of a stage (32 k; us, on
   // 961 x 4864 x 896, 961 x 896 x 4864, 4096^3 and 2048 x 14336 x 4096), plus the bytes of the
   // outputs and, for K slices, of the partial tiles and their reduce at 4 TB/s and its launch.
@@ -463,22 +463,19 @@ PackedPlan plan_packed(int m, int rows, int K, bool sp, bool pairs) {
   const Shape* sh = sp ? f32 : bf;
   const int ns = sp ? 4 : 3, steps = (K + 31) / 32;
   const double out_us = (double)m * rows * 4 / 4e6;
+  const int first = splits ? splits : 1, last = splits ? splits : pairs ? 1 : 8;
   PackedPlan best;
-  double best_us = 1e30;
+  best.us = 1e30;
   for (int i = 0; i < ns; ++i) {
     if (pairs && sh[i].t == PackedTile::k192x128) continue;   // three 32-row groups per wave
     const long tiles = (long)((m + sh[i].bm - 1) / sh[i].bm) * ((rows + sh[i].bn - 1) / sh[i].bn);
-    for (int sp_n = 1; sp_n <= (pairs ? 1 : 8); ++sp_n) {
+    for (int sp_n = first; sp_n <= last; ++sp_n) {
       const int per = (steps + sp_n - 1) / sp_n;
-      if (sp_n > 1 && (per < 4 || (steps + per - 1) / per != sp_n || (double)sp_n * rows * m * 4 > (32 << 20))) continue;
+      if (!splits && sp_n > 1 &&
+          (per < 4 || (steps + per - 1) / per != sp_n || (double)sp_n * rows * m * 4 > (32 << 20))) continue;
       double us = (double)((tiles * sp_n + 255) / 256) * per * sh[i].us + out_us * sp_n;
       if (sp_n > 1) us += 2.0 + out_us * (sp_n + 1);
-      if (us < best_us) {
-        best_us = us;
-        best.tile = sh[i].t;
-        best.splits = sp_n;
-        best.steps_per_split = per;
-      }
+      if (us < best.us) best = {sh[i].t, sp_n, per, us};
     }
   }
   return best;

@@ -101,6 +101,24 @@ def test_operands_in_pieces():
     q.close()
 
 
+@pytest.mark.parametrize("t,m,n,rows,pieces", [(rehip.Q4_0, 28672, 1024, 1024, True), (rehip.F16, 4096, 4096, 512, True),
+                                               (rehip.Q4_0, 4096, 4096, 512, False),
+                                               (rehip.Q4_0, 2048, 8192, 1024, False),
+                                               (rehip.F16, 2048, 8192, 1024, False)])
+def test_pieces_only_where_they_fill_the_gpu(t, m, n, rows, pieces):
+    """The no-allocation entry point with operands beyond its scratch: in pieces of the same bits, or the
+    unpacked GEMM's bits where the pieces would be small or the rows few."""
+    rng = np.random.default_rng(m)
+    q = rehip.QMat.from_bytes(t, weights(rng, t, m, n), m, n)
+    dx = B.from_array(synth.activations(rng, rows, n))
+    got = run(q, dx, rows, m, rehip.MODE_F32, "matmul_noalloc_dev")
+    with pytest.MonkeyPatch.context() as mp:
+        if not pieces:
+            mp.setenv("REHIP_GEMM_PACKED", "0")
+        assert np.array_equal(run(q, dx, rows, m, rehip.MODE_F32), got)
+    q.close()
+
+
 def test_streams_and_capture():
     """More live streams than workspaces, two matrices in turn and no synchronisation in between; then a
     captured call (the tiled GEMM) replayed between eager ones."""
