@@ -233,9 +233,10 @@ int re_kv_append_dev(const float *d_k, const float *d_v, size_t rows, size_t kv_
 /* Causal GQA attention of rows x n_heads x head_dim queries at positions *d_pos + r over cache
  * rows 0..position (forward.rs:232-277, 437-470); max_seq <= 32768 cache rows, positions are
  * clamped to them. Output rows x n_heads x head_dim. Rows >= 8 with head_dim 32, 64, 96 or 128 run as
- * f32 MFMA flash attention; fewer rows use d_work (re_attention_work_bytes bytes; NULL = one workgroup
- * per head and row, slower for long caches) to split the cache over workgroups. Buffers are
- * 16-byte aligned. */
+ * f32 MFMA flash attention, except that up to 400, 600 and 900 (row, head) pairs of head_dim 32, 96 and
+ * 128, like fewer rows, use d_work (re_attention_work_bytes bytes; NULL = no such exception, and fewer
+ * rows run one workgroup per head and row, slower for long caches) to split the cache over workgroups.
+ * Buffers are 16-byte aligned. */
 size_t re_attention_work_bytes(size_t rows, size_t n_heads, size_t head_dim, size_t max_seq);
 int re_attention_dev(const float *d_q, const float *d_kcache, const float *d_vcache, size_t rows,
                      size_t n_heads, size_t n_kv_heads, size_t head_dim, size_t max_seq,

@@ -1039,7 +1039,14 @@ hipError_t launch_attention(const float* q, const float* kc, const float* vc, in
   // workgroup per (head, row) with no workspace 29 us, and the gap widens with the rows (300 rows of 8
   // heads of 32: 9 against 83 us). Other head sizes (up to 256) do not tile by 32, or do not fit the
   // registers; a cache of 2 GiB or more does not fit the 32-bit offsets. They keep the kernels below.
-  if (rows >= 8 && hd % 32 == 0 && hd <= 128 && (size_t)max_seq * kv_heads * hd * 4 < (1ull << 31)) {
+  // With a workspace, few (row, head) pairs go to the split kernel: the matrix cores serve 32 pairs of a kv
+  // head by one workgroup, which walks all their keys, so both times grow with the keys alike and the
+  // line is a number of pairs (us split / matrix cores, 14 / 2 heads of 128 in a cache of 4096: 8 rows at 4088
+  // 30 / 154, 64 rows at 4032 167 / 156; 24 / 8 heads of 96: about 600 pairs; 32 / 32 heads of 32: about 400). A
+  // large cache with little in it costs the split kernel its empty splits (8 rows at 0 of 32768: 15 / 9).
+  const int split_pairs = hd == 128 ? 900 : hd == 96 ? 600 : hd == 32 ? 400 : 0;
+  const bool few = work && (long)rows * heads <= split_pairs;
+  if (rows >= 8 && !few && hd % 32 == 0 && hd <= 128 && (size_t)max_seq * kv_heads * hd * 4 < (1ull << 31)) {
     const int grp = heads / kv_heads;
     const dim3 grid((unsigned)(((size_t)rows * grp + kAttnMfmaVecs - 1) / kAttnMfmaVecs * kv_heads));
     auto* k = hd == 32   ? attention_mfma_kernel<32>

@@ -48,6 +48,27 @@ def test_edges(hd, rows, pos, heads, kv_heads, max_seq):
     np.testing.assert_allclose(run(q, kc, vc, pos), want, rtol=0, atol=3e-5 * np.abs(want).max())
 
 
+@pytest.mark.parametrize("hd,pairs", [(32, 400), (96, 600), (128, 900)])
+def test_few_pairs_with_a_workspace_split_the_cache(hd, pairs):
+    """On both sides of the line, with and without a workspace: the same attention, and the workspace used
+    (its splits written) up to the line only."""
+    heads, kv_heads, max_seq, pos = 10, 2, 300, 200
+    rng = np.random.default_rng(hd)
+    kc, vc = (rng.standard_normal((max_seq, kv_heads, hd)).astype(np.float32) for _ in range(2))
+    for rows in (8, pairs // heads, pairs // heads + 1):
+        q = 2 * rng.standard_normal((rows, heads, hd)).astype(np.float32)
+        wb = rehip.attention_work_bytes(rows, heads, hd, max_seq)
+        work, ctx = B.from_array(np.full(wb // 4, 7.5, np.float32)), B(q.nbytes)
+        rehip.attention_dev(B.from_array(q), B.from_array(kc), B.from_array(vc), rows, heads, kv_heads, hd, max_seq,
+                            B.from_array(np.array([pos], np.int32)), ctx, work=work, work_bytes=wb)
+        hip.synchronize()
+        assert np.any(work.download(np.float32, wb // 4) != 7.5) == (rows * heads <= pairs)
+        want = reference(q, kc, vc, pos, kv_heads)
+        tol = 3e-5 * np.abs(want).max()
+        np.testing.assert_allclose(ctx.download(np.float32, q.size).reshape(q.shape), want, rtol=0, atol=tol)
+        np.testing.assert_allclose(run(q, kc, vc, pos), want, rtol=0, atol=tol)
+
+
 @pytest.mark.parametrize("hd", [64, 128])
 @pytest.mark.parametrize("bad", [np.inf, np.nan])
 def test_hidden_rows_may_hold_anything(hd, bad):
