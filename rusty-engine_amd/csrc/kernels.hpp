@@ -158,19 +158,16 @@ hipError_t launch_gemm(uint32_t type, int mode, const GemmArgs& a, int ntasks, G
                        hipStream_t s);
 // GEMM over packed bf16 operands (packed.hip): one launch packs a range of weight rows and
 // activation rows as MFMA fragments, then the GEMM runs on them. KS: k steps of 16 per row,
-// ceil(K / 32) * 2. An operand of r rows takes packed_bytes(r, KS) per plane (two planes in f32 mode).
+// ceil(K / 32) * 2. An operand of r rows takes KS * 32 bytes per row and plane (two planes in f32 mode).
 constexpr int kPackedRows = 256;          // packed operands are padded to whole tiles of this many rows
-inline size_t packed_bytes(size_t rows, int KS) {
-  return (rows + kPackedRows - 1) / kPackedRows * kPackedRows * (size_t)KS * 32;
-}
 struct PackArgs {
   const void* W;           // the whole matrix: tiled slabs, or row-major F32 / F16 / BF16
   int w_row0, w_rows;      // weight rows to pack (w_row0 a multiple of 64; w_rows 0: none)
   int K, KS, KB;
   const float* x;          // activation rows to pack (x_rows 0: none)
   int x_rows;
-  const void* W2 = nullptr;   // quantized only: a second matrix of the same shape; groups of 32 rows of W
-                              // and W2 then alternate in Wp (w_row0 0, w_rows a multiple of 32)
+  const void* W2 = nullptr;   // quantized only: a second matrix of the same shape (it may be W); groups of 32
+                              // rows of W and W2 then alternate in Wp (w_rows a multiple of 32)
   uint8_t *Wp, *Xp;        // packed planes; the remainders' planes w_lo / x_lo bytes further
   size_t w_lo, x_lo;
   int w_groups;            // set by launch_pack

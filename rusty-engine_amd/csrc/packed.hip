@@ -178,24 +178,25 @@ __global__ __launch_bounds__(256) void pack_kernel(PackArgs p) {
 }
 
 // The GEMM. A workgroup of WM x WN waves computes BM weight rows x BN activation rows in stages of
-// 32 k (two fragments deep), NB stage buffers in LDS filled by DMA up to NB - 1 stages ahead.
-// A wave's body for stage s: read its second k step, multiply the first (read one half stage
-// earlier), wait for stage s + 1 and the workgroup, refill this stage's buffer with stage s + NB,
-// read the first k step of stage s + 1, multiply the second. So one barrier per stage, with MFMAs
-// on both sides of it, and no read waits for its own stage's copy.
+// 32 k (two fragments deep), with NB stage buffers in LDS filled by DMA and the operands of two stages in
+// registers. A wave's body for stage s, whose operands it has read: wait for its own copies of stage s + 1
+// and for the workgroup (all waves have then read stage s), then multiply stage s, reading the operands of
+// stage s + 1 among the first half of the MFMAs and refilling stage s's buffer with stage s + NB among
+// the second. So one barrier per stage, copies that have NB - 1 stages to land, and no read that waits for
+// a copy or MFMA that waits for its stage's reads.
 // The activations are the A operand (rows of D): a lane then holds one weight row's column of D,
 // and a store instruction writes two whole 128-byte runs of two output rows.
 // SW: the SwiGLU epilogue. The weights are the A operand, so a lane holds one activation row and runs of
 // four consecutive weight rows, and writes h as 8-byte halves of the next GEMM's fragment units.
-template <int BM, int BN, int WM, int WN, int KK, int NB, bool SP, bool SW>
+template <int BM, int BN, int WM, int WN, int NB, bool SP, bool SW>
 __global__ __launch_bounds__(WM* WN * 64) void packed_gemm_kernel(PackedGemmArgs p) {
-  constexpr int NWAVE = WM * WN;
+  constexpr int NWAVE = WM * WN, KK = 2;                        // k steps of 16 per stage
   constexpr int TM = BM / WM / 32, TN = BN / WN / 32;
   constexpr int P = SP ? 2 : 1;
   constexpr int WQ = BM / 32 * KK * P, XQ = BN / 32 * KK * P;   // 1 KiB pieces per stage
   constexpr int NI = (WQ + XQ) / NWAVE;
   constexpr int SB = (WQ + XQ) * 1024;
-  static_assert((WQ + XQ) % NWAVE == 0 && NB >= 2 && (KK == 2 || KK == 4) && NB * SB <= (int)kMaxLdsBytes, "stage split");
+  static_assert((WQ + XQ) % NWAVE == 0 && NB >= 2 && NB * SB <= (int)kMaxLdsBytes, "stage split");
   __shared__ __attribute__((aligned(1024))) uint8_t smem[NB * SB];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -374,11 +375,11 @@ __global__ __launch_bounds__(WM* WN * 64) void packed_gemm_kernel(PackedGemmArgs
   }
 }
 
-template <int BM, int BN, int WM, int WN, int KK, int NB, bool SP, bool SW = false>
+template <int BM, int BN, int WM, int WN, int NB, bool SP, bool SW = false>
 hipError_t launch_shape(const PackedGemmArgs& a, hipStream_t s, hipEvent_t done) {
   const int total = ((a.m + BM - 1) / BM) * ((a.N + BN - 1) / BN) * a.splits;
   const int grid = (total + 7) / 8 * 8;
-  auto* k = packed_gemm_kernel<BM, BN, WM, WN, KK, NB, SP, SW>;
+  auto* k = packed_gemm_kernel<BM, BN, WM, WN, NB, SP, SW>;
   if (done) hipExtLaunchKernelGGL(k, dim3((unsigned)grid), dim3(WM * WN * 64), 0, s, nullptr, done, 0, a);
   else hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(WM * WN * 64), 0, s, a);
   return hipGetLastError();
@@ -422,31 +423,31 @@ hipError_t launch_packed_gemm(const PackedGemmArgs& a, PackedTile tile, bool sp,
     if (a.splits != 1) return hipErrorInvalidValue;
     if (sp) {
       switch (tile) {
-        case PackedTile::k256x128: return launch_shape<256, 128, 4, 2, 2, 3, true, true>(a, s, done);
-        case PackedTile::k128x128: return launch_shape<128, 128, 2, 2, 2, 4, true, true>(a, s, done);
-        case PackedTile::k128x64: return launch_shape<128, 64, 2, 2, 2, 3, true, true>(a, s, done);
+        case PackedTile::k256x128: return launch_shape<256, 128, 4, 2, 3, true, true>(a, s, done);
+        case PackedTile::k128x128: return launch_shape<128, 128, 2, 2, 4, true, true>(a, s, done);
+        case PackedTile::k128x64: return launch_shape<128, 64, 2, 2, 3, true, true>(a, s, done);
         default: return hipErrorInvalidValue;
       }
     }
     switch (tile) {
-      case PackedTile::k256x256: return launch_shape<256, 256, 2, 4, 2, 4, false, true>(a, s, done);
-      case PackedTile::k128x128: return launch_shape<128, 128, 2, 2, 2, 4, false, true>(a, s, done);
+      case PackedTile::k256x256: return launch_shape<256, 256, 2, 4, 4, false, true>(a, s, done);
+      case PackedTile::k128x128: return launch_shape<128, 128, 2, 2, 4, false, true>(a, s, done);
       default: return hipErrorInvalidValue;
     }
   }
   if (sp) {
     switch (tile) {
-      case PackedTile::k256x128: return launch_shape<256, 128, 4, 2, 2, 3, true>(a, s, done);
-      case PackedTile::k192x128: return launch_shape<192, 128, 2, 2, 2, 4, true>(a, s, done);
-      case PackedTile::k128x128: return launch_shape<128, 128, 2, 2, 2, 4, true>(a, s, done);
-      case PackedTile::k128x64: return launch_shape<128, 64, 2, 2, 2, 3, true>(a, s, done);
+      case PackedTile::k256x128: return launch_shape<256, 128, 4, 2, 3, true>(a, s, done);
+      case PackedTile::k192x128: return launch_shape<192, 128, 2, 2, 4, true>(a, s, done);
+      case PackedTile::k128x128: return launch_shape<128, 128, 2, 2, 4, true>(a, s, done);
+      case PackedTile::k128x64: return launch_shape<128, 64, 2, 2, 3, true>(a, s, done);
       default: return hipErrorInvalidValue;
     }
   }
   switch (tile) {
-    case PackedTile::k256x256: return launch_shape<256, 256, 2, 4, 2, 4, false>(a, s, done);
-    case PackedTile::k192x128: return launch_shape<192, 128, 2, 2, 2, 4, false>(a, s, done);
-    case PackedTile::k128x128: return launch_shape<128, 128, 2, 2, 2, 4, false>(a, s, done);
+    case PackedTile::k256x256: return launch_shape<256, 256, 2, 4, 4, false>(a, s, done);
+    case PackedTile::k192x128: return launch_shape<192, 128, 2, 2, 4, false>(a, s, done);
+    case PackedTile::k128x128: return launch_shape<128, 128, 2, 2, 4, false>(a, s, done);
     default: return hipErrorInvalidValue;
   }
 }

@@ -71,8 +71,8 @@ def test_against_f64(t, td, d, ff, rows, mode, monkeypatch):
 @pytest.mark.parametrize("mode", MODES)
 @pytest.mark.parametrize("rows", [1, 5, 100, 300, 700])
 def test_equals_separate_calls(mode, rows):
-    """The default rule on both sides of its line; K of one slice, so every product's sums run in the
-    same order: the same bits where the separate products are packed too or nothing is."""
+    """The default rule on both sides of its line: within the roundings of the separate calls, and their
+    bits below 64 rows, where the block runs them."""
     d, ff = 224, 3072
     rng = np.random.default_rng(rows)
     w = matrices(rng, rehip.Q4_0, rehip.Q4_0, d, ff)
