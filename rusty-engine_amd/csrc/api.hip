@@ -543,17 +543,19 @@ struct PackedCall {
   uint32_t type;
   const void* W;
   int m, K, KB, rows;
-  bool sp;
+  bool sp;                                        // f32 mode
   PackedPlan plan;
-  size_t row_bytes() const { return (size_t)(K + 31) / 32 * 64 * (sp ? 2 : 1); }
+  int w_planes() const { return sp && type != 30 ? 2 : 1; }   // (BF16 weights leave no remainder)
+  int x_planes() const { return sp ? 2 : 1; }
+  int products() const { return w_planes() + x_planes() - 1; }
+  size_t plane_bytes() const { return (size_t)(K + 31) / 32 * 64; }   // of a row
+  size_t w_row() const { return plane_bytes() * w_planes(); }
+  size_t x_row() const { return plane_bytes() * x_planes(); }
   size_t partial_bytes() const {
     return plan.splits > 1 ? ((size_t)plan.splits * rows * m * sizeof(float) + 255) / 256 * 256 : 0;
   }
   // bytes that hold both operands whole, at most `cap`
-  size_t want(size_t cap) const {
-    const size_t all = partial_bytes() + (pad(m) + pad(rows)) * row_bytes();
-    return std::min(all, cap);
-  }
+  size_t want(size_t cap) const { return std::min(partial_bytes() + pad(m) * w_row() + pad(rows) * x_row(), cap); }
   static size_t pad(size_t r) { return (r + kPackedRows - 1) / kPackedRows * kPackedRows; }
 };
 
@@ -604,8 +606,8 @@ bool packed_call(uint32_t type, const void* W, size_t m, size_t K, size_t KB, co
   c->KB = (int)KB;
   c->rows = (int)rows;
   c->sp = sp;
-  if (2 * kPackedRows * c->row_bytes() > kScratchBytes / 2) return false;
-  c->plan = plan_packed((int)m, (int)rows, (int)K, sp);
+  if (2 * kPackedRows * c->x_row() > kScratchBytes / 2) return false;
+  c->plan = plan_packed((int)m, (int)rows, (int)K, c->products());
   return true;
 }
 
@@ -619,15 +621,15 @@ bool dense_packed(const re_qmat* q, const float* d_x, size_t rows, int mode, Pac
 // Rows of each operand packed at a time in a workspace of ws_bytes (whole operands if they fit); false: too
 // small for any.
 bool packed_pieces(const PackedCall& c, size_t ws_bytes, size_t* mc, size_t* nc) {
-  const size_t rb = c.row_bytes(), part = c.partial_bytes();
+  const size_t wr = c.w_row(), xr = c.x_row(), part = c.partial_bytes();
   *mc = PackedCall::pad(c.m);
   *nc = PackedCall::pad(c.rows);
   if (part >= ws_bytes) return false;
-  const size_t most = (ws_bytes - part) / rb;
-  if (*mc + *nc <= most) return true;
-  *nc = std::min(*nc, std::max<size_t>(kPackedRows, most / 2 / kPackedRows * kPackedRows));
-  if (*nc >= most) return false;
-  *mc = std::min(*mc, (most - *nc) / kPackedRows * kPackedRows);
+  const size_t avail = ws_bytes - part;
+  if (*mc * wr + *nc * xr <= avail) return true;
+  *nc = std::min(*nc, std::max<size_t>(kPackedRows, avail / 2 / xr / kPackedRows * kPackedRows));
+  if (*nc * xr >= avail) return false;
+  *mc = std::min(*mc, (avail - *nc * xr) / wr / kPackedRows * kPackedRows);
   return *mc > 0;
 }
 
@@ -650,21 +652,21 @@ bool pieces_pay(const PackedCall& c, size_t ws_bytes) {
   int pieces = 0;
   for (size_t n0 = 0; n0 < (size_t)c.rows; n0 += nc)
     for (size_t m0 = 0; m0 < (size_t)c.m; m0 += mc, ++pieces)
-      us += plan_packed((int)std::min(mc, c.m - m0), (int)std::min(nc, c.rows - n0), c.K, c.sp, false, c.plan.splits).us;
+      us += plan_packed((int)std::min(mc, c.m - m0), (int)std::min(nc, c.rows - n0), c.K, c.products(), false, c.plan.splits).us;
   return us + 5.0 * (pieces - 1) <= (dense ? 2.0 : 1.4) * c.plan.us;
 }
 
 // done: carried by the last launch (nullptr: none)
 int packed_enqueue(const PackedCall& c, const float* d_x, float* d_y, void* ws, size_t ws_bytes, hipStream_t s,
                    hipEvent_t done = nullptr) {
-  const size_t rb = c.row_bytes(), part = c.partial_bytes(), mp = PackedCall::pad(c.m);
+  const size_t wr = c.w_row(), xr = c.x_row(), part = c.partial_bytes(), mp = PackedCall::pad(c.m);
   size_t mc, nc;
   if (!packed_pieces(c, ws_bytes, &mc, &nc))
     return fail(RE_ERR_SIZE, "packed GEMM workspace of %zu bytes is too small", ws_bytes);
-  const int KS = (c.K + 31) / 32 * 2, planes = c.sp ? 2 : 1;
+  const int KS = (c.K + 31) / 32 * 2;
   float* partial = c.plan.splits > 1 ? (float*)ws : nullptr;
   uint8_t* wp = (uint8_t*)ws + part;
-  uint8_t* xp = wp + mc * rb;
+  uint8_t* xp = wp + mc * wr;
   for (size_t n0 = 0; n0 < (size_t)c.rows; n0 += nc) {
     const size_t rows = std::min(nc, c.rows - n0);
     for (size_t m0 = 0; m0 < (size_t)c.m; m0 += mc) {
@@ -680,14 +682,14 @@ int packed_enqueue(const PackedCall& c, const float* d_x, float* d_y, void* ws, 
       pa.x_rows = m0 ? 0 : (int)rows;
       pa.Wp = wp;
       pa.Xp = xp;
-      pa.w_lo = mc * rb / planes;
-      pa.x_lo = nc * rb / planes;
+      pa.w_lo = mc * c.plane_bytes();             // (unused where there is one plane)
+      pa.x_lo = nc * c.plane_bytes();
       HIP_TRY(launch_pack(c.type, pa, c.sp, s));
       PackedGemmArgs a{};
       a.Wp = wp;
       a.Xp = xp;
-      a.w_bytes = (uint32_t)(mc * rb);
-      a.x_bytes = (uint32_t)(nc * rb);
+      a.w_bytes = (uint32_t)(mc * wr);
+      a.x_bytes = (uint32_t)(nc * xr);
       a.w_lo = (uint32_t)pa.w_lo;
       a.x_lo = (uint32_t)pa.x_lo;
       a.Y = d_y + n0 * c.m + m0;
@@ -702,9 +704,9 @@ int packed_enqueue(const PackedCall& c, const float* d_x, float* d_y, void* ws, 
       // a piece's own tile, the whole product's K slices: the same sums
       const PackedTile tile = mr == (size_t)c.m && rows == (size_t)c.rows
                                   ? c.plan.tile
-                                  : plan_packed((int)mr, (int)rows, c.K, c.sp, false, c.plan.splits).tile;
+                                  : plan_packed((int)mr, (int)rows, c.K, c.products(), false, c.plan.splits).tile;
       const bool last = n0 + nc >= (size_t)c.rows && m0 + mc >= (size_t)c.m;
-      HIP_TRY(launch_packed_gemm(a, tile, c.sp, s, last && !partial ? done : nullptr));
+      HIP_TRY(launch_packed_gemm(a, tile, c.products(), s, last && !partial ? done : nullptr));
     }
   }
   if (partial) HIP_TRY(launch_gemm_reduce(partial, d_y, (size_t)c.rows * c.m, c.plan.splits, s, nullptr, done));
@@ -778,10 +780,10 @@ int packed_ffn(re_qmat* gate, re_qmat* up, re_qmat* down, const float* d_x, size
   if (knob != 2 && !packed_ffn_pays(ff, gate->g.n, rows, sp)) return RE_OK;
   PackedCall c1{gate->g.type, gate->d_w, (int)(2 * ff), (int)gate->g.n, (int)gate->g.kb, (int)rows, sp, {}};
   PackedCall c2{down->g.type, down->d_w, (int)d, (int)ff, (int)down->g.kb, (int)rows, sp, {}};
-  c1.plan = plan_packed(c1.m, c1.rows, c1.K, sp, true);
-  c2.plan = plan_packed(c2.m, c2.rows, c2.K, sp);
+  c1.plan = plan_packed(c1.m, c1.rows, c1.K, c1.products(), true);
+  c2.plan = plan_packed(c2.m, c2.rows, c2.K, c2.products());
   // the K-slice partials, x, h, and a region for packed weights: pieces of gate and up, then of down
-  const size_t rb1 = c1.row_bytes(), rb2 = c2.row_bytes(), part = c2.partial_bytes();
+  const size_t rb1 = c1.x_row(), rb2 = c2.x_row(), part = c2.partial_bytes();
   const size_t xb = PackedCall::pad(rows) * rb1, hb = PackedCall::pad(rows) * rb2, fixed = part + xb + hb;
   if (fixed + kPackedWsBytes / 8 > kPackedWsBytes) return RE_OK;
   const size_t region = std::min(std::max(PackedCall::pad(2 * ff) * rb1, PackedCall::pad(d) * rb2), kPackedWsBytes - fixed);
@@ -829,7 +831,7 @@ int packed_ffn(re_qmat* gate, re_qmat* up, re_qmat* down, const float* d_x, size
       a.Hp = hp + f0 / 16 * 1024;
       a.h_lo = (uint32_t)(hb / planes);
       a.KSh = KS2;
-      HIP_TRY(launch_packed_gemm(a, c1.plan.tile, sp, s));
+      HIP_TRY(launch_packed_gemm(a, c1.plan.tile, c1.products(), s));
     }
     float* partial = c2.plan.splits > 1 ? (float*)ws : nullptr;
     for (size_t m0 = 0; m0 < d; m0 += dc) {
@@ -860,7 +862,7 @@ int packed_ffn(re_qmat* gate, re_qmat* up, re_qmat* down, const float* d_x, size
       b.splits = c2.plan.splits;
       b.steps_per_split = c2.plan.steps_per_split;
       b.add = partial || !d_add ? nullptr : d_add + m0;   // else in the reduce
-      HIP_TRY(launch_packed_gemm(b, c2.plan.tile, sp, s, !partial && m0 + dc >= d ? done : nullptr));
+      HIP_TRY(launch_packed_gemm(b, c2.plan.tile, c2.products(), s, !partial && m0 + dc >= d ? done : nullptr));
     }
     if (partial) HIP_TRY(launch_gemm_reduce(partial, d_y, rows * d, c2.plan.splits, s, d_add, done));
     return RE_OK;

@@ -158,7 +158,8 @@ hipError_t launch_gemm(uint32_t type, int mode, const GemmArgs& a, int ntasks, G
                        hipStream_t s);
 // GEMM over packed bf16 operands (packed.hip): one launch packs a range of weight rows and
 // activation rows as MFMA fragments, then the GEMM runs on them. KS: k steps of 16 per row,
-// ceil(K / 32) * 2. An operand of r rows takes KS * 32 bytes per row and plane (two planes in f32 mode).
+// ceil(K / 32) * 2. An operand takes KS * 32 bytes per row and plane; in f32 mode there
+// are two planes, of BF16 weights one.
 constexpr int kPackedRows = 256;          // packed operands are padded to whole tiles of this many rows
 struct PackArgs {
   const void* W;           // the whole matrix: tiled slabs, or row-major F32 / F16 / BF16
@@ -172,7 +173,7 @@ struct PackArgs {
   size_t w_lo, x_lo;
   int w_groups;            // set by launch_pack
 };
-// sp: f32 mode (hi and lo planes). n % 8 == 0 and 16-byte aligned rows for row-major weights and x.
+// sp: f32 mode. n % 8 == 0 and 16-byte aligned rows for row-major weights and x.
 hipError_t launch_pack(uint32_t type, PackArgs a, bool sp, hipStream_t s);
 enum class PackedTile { k256x256, k256x128, k192x128, k128x128, k128x64 };   // weight rows x activation rows
 struct PackedPlan {
@@ -180,9 +181,10 @@ struct PackedPlan {
   int splits = 1, steps_per_split = 1;
   double us = 0;           // the estimate it was chosen by
 };
-// pairs: the SwiGLU epilogue (one K slice, whole gate / up pairs per wave); splits: the K slices of a
-// piece of a larger product (0: free)
-PackedPlan plan_packed(int m, int rows, int K, bool sp, bool pairs = false, int splits = 0);
+// products: MFMAs per pair of operands, 1 in bf16 mode, 3 in f32 mode, 2 there for BF16 weights; pairs: the
+// SwiGLU epilogue (one K slice, whole gate / up pairs per wave; products 1 and 3); splits: the K slices of
+// a piece of a larger product (0: free)
+PackedPlan plan_packed(int m, int rows, int K, int products, bool pairs = false, int splits = 0);
 struct PackedGemmArgs {
   const uint8_t *Wp, *Xp;
   uint32_t w_bytes, x_bytes;   // all planes
@@ -200,7 +202,7 @@ struct PackedGemmArgs {
   int KSh = 0;
 };
 // done: an event that the launch's end completes (nullptr: none)
-hipError_t launch_packed_gemm(const PackedGemmArgs& a, PackedTile tile, bool sp, hipStream_t s,
+hipError_t launch_packed_gemm(const PackedGemmArgs& a, PackedTile tile, int products, hipStream_t s,
                               hipEvent_t done = nullptr);
 // Few-row dense GEMM (skinny.hip): Y[N x m] = X[N x K] W^T for N <= 64 rows of f32 X, a 64-row
 // weight tile and a K slice of blocks_per_split whole blocks per workgroup; splits > 1 writes

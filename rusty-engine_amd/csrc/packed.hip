@@ -13,9 +13,10 @@
 // to LDS in contiguous 1 KiB pieces. K past the row is zero in both operands; rows past the
 // matrix are not written (they feed outputs that are not stored).
 //
-// f32 mode (SP): a second plane of each operand holds the bf16 rounding of what the first leaves,
-// and every product is w_hi x_hi + w_hi x_lo + w_lo x_hi in f32 accumulators, each term within
-// 2^-16 relative, as in the tiled GEMM.
+// f32 mode: a second plane of each operand holds the bf16 rounding of what the first leaves, and every
+// product is w_hi x_hi + w_hi x_lo + w_lo x_hi in f32 accumulators, each term within 2^-16 relative, as in
+// the tiled GEMM. BF16 weights leave nothing: one plane and two products, w x_hi + w x_lo. NP: products
+// per pair of operands (1 in bf16 mode, 3 or 2 in f32 mode).
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
@@ -160,8 +161,8 @@ __global__ __launch_bounds__(256) void pack_kernel(PackArgs p) {
       const int g = job / kcs;
       if (32 * g >= p.w_rows) return;
       constexpr size_t ES = T == 0 ? 4 : 2;
-      pack_rows<T, SP>((const uint8_t*)p.W + (size_t)p.w_row0 * p.K * ES, p.w_rows, p.K, p.KS, g, job - g * kcs, p.Wp,
-                       p.w_lo);
+      pack_rows<T, SP && T != 30>((const uint8_t*)p.W + (size_t)p.w_row0 * p.K * ES, p.w_rows, p.K, p.KS, g,
+                                  job - g * kcs, p.Wp, p.w_lo);
     } else {
       const int nch = p.KB * Blk<(int)T>::NCH;
       const int t = job / nch, nt = (p.w_rows + 63) / 64;
@@ -188,12 +189,12 @@ __global__ __launch_bounds__(256) void pack_kernel(PackArgs p) {
 // and a store instruction writes two whole 128-byte runs of two output rows.
 // SW: the SwiGLU epilogue. The weights are the A operand, so a lane holds one activation row and runs of
 // four consecutive weight rows, and writes h as 8-byte halves of the next GEMM's fragment units.
-template <int BM, int BN, int WM, int WN, int NB, bool SP, bool SW>
+template <int BM, int BN, int WM, int WN, int NB, int NP, bool SW>
 __global__ __launch_bounds__(WM* WN * 64) void packed_gemm_kernel(PackedGemmArgs p) {
   constexpr int NWAVE = WM * WN, KK = 2;                        // k steps of 16 per stage
   constexpr int TM = BM / WM / 32, TN = BN / WN / 32;
-  constexpr int P = SP ? 2 : 1;
-  constexpr int WQ = BM / 32 * KK * P, XQ = BN / 32 * KK * P;   // 1 KiB pieces per stage
+  constexpr int PX = NP > 1 ? 2 : 1, PW = NP == 3 ? 2 : 1;      // planes
+  constexpr int WQ = BM / 32 * KK * PW, XQ = BN / 32 * KK * PX;  // 1 KiB pieces per stage
   constexpr int NI = (WQ + XQ) / NWAVE;
   constexpr int SB = (WQ + XQ) * 1024;
   static_assert((WQ + XQ) % NWAVE == 0 && NB >= 2 && NB * SB <= (int)kMaxLdsBytes, "stage split");
@@ -249,11 +250,12 @@ __global__ __launch_bounds__(WM* WN * 64) void packed_gemm_kernel(PackedGemmArgs
       for (int r = 0; r < 16; ++r) acc[j][i][r] = 0.0f;
 
   // a whole stage's operands
-  struct Ops { bf16x8_t w[KK][P][TM], x[KK][P][TN]; };
-  constexpr int NR = KK * P * (TM + TN);              // fragment reads per stage
-  constexpr int NM = KK * TM * TN * (SP ? 3 : 1);     // MFMAs per stage
+  struct Ops { bf16x8_t w[KK][PW][TM], x[KK][PX][TN]; };
+  constexpr int NR1 = PW * TM + PX * TN, NR = KK * NR1;   // fragment reads per k step and stage
+  constexpr int NM = KK * TM * TN * NP;                   // MFMAs per stage
+  // per k step: the first planes' activations and weights, then the second planes'
   auto read = [&](const uint8_t* buf, Ops& o, int i) {
-    const int kk = i / (P * (TM + TN)), pl = i / (TM + TN) % P, f = i % (TM + TN);
+    const int kk = i / NR1, pl = i % NR1 / (TM + TN), f = i % NR1 % (TM + TN);
     if (f < TN)
       o.x[kk][pl][f] = *reinterpret_cast<const bf16x8_t*>(
           buf + (WQ + pl * (BN / 32 * KK) + KK * (wn * TN + f) + kk) * 1024 + lane * 16);
@@ -261,10 +263,10 @@ __global__ __launch_bounds__(WM* WN * 64) void packed_gemm_kernel(PackedGemmArgs
       o.w[kk][pl][f - TN] = *reinterpret_cast<const bf16x8_t*>(
           buf + (pl * (BM / 32 * KK) + KK * (wm * TM + f - TN) + kk) * 1024 + lane * 16);
   };
-  // MFMA i of a stage: per k step the w_hi x_hi products, then (f32 mode) w_hi x_lo and w_lo x_hi
+  // MFMA i of a stage: per k step the w_hi x_hi products, then w_hi x_lo and w_lo x_hi
   auto mma = [&](const Ops& o, int i) {
-    const int kk = i / (NM / KK), term = i / (TM * TN) % (SP ? 3 : 1), m = i / TN % TM, n = i % TN;
-    const bf16x8_t x = o.x[kk][SP && term == 1][n], w = o.w[kk][SP && term == 2][m];
+    const int kk = i / (NM / KK), term = i / (TM * TN) % NP, m = i / TN % TM, n = i % TN;
+    const bf16x8_t x = o.x[kk][term == 1][n], w = o.w[kk][term == 2][m];
     acc[n][m] = SW ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(w, x, acc[n][m], 0, 0, 0)
                    : __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, w, acc[n][m], 0, 0, 0);
   };
@@ -332,7 +334,7 @@ __global__ __launch_bounds__(WM* WN * 64) void packed_gemm_kernel(PackedGemmArgs
           }
           uint8_t* d = p.Hp + unit_off(x, k0 + 8 * q, p.KSh) + 8 * (lane >> 5);
           *reinterpret_cast<bf16x4_t*>(d) = hi;
-          if constexpr (SP) *reinterpret_cast<bf16x4_t*>(d + p.h_lo) = lo;
+          if constexpr (NP > 1) *reinterpret_cast<bf16x4_t*>(d + p.h_lo) = lo;
         }
       }
     }
@@ -375,11 +377,11 @@ __global__ __launch_bounds__(WM* WN * 64) void packed_gemm_kernel(PackedGemmArgs
   }
 }
 
-template <int BM, int BN, int WM, int WN, int NB, bool SP, bool SW = false>
+template <int BM, int BN, int WM, int WN, int NB, int NP, bool SW = false>
 hipError_t launch_shape(const PackedGemmArgs& a, hipStream_t s, hipEvent_t done) {
   const int total = ((a.m + BM - 1) / BM) * ((a.N + BN - 1) / BN) * a.splits;
   const int grid = (total + 7) / 8 * 8;
-  auto* k = packed_gemm_kernel<BM, BN, WM, WN, NB, SP, SW>;
+  auto* k = packed_gemm_kernel<BM, BN, WM, WN, NB, NP, SW>;
   if (done) hipExtLaunchKernelGGL(k, dim3((unsigned)grid), dim3(WM * WN * 64), 0, s, nullptr, done, 0, a);
   else hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(WM * WN * 64), 0, s, a);
   return hipGetLastError();
@@ -418,41 +420,39 @@ hipError_t launch_pack(uint32_t type, PackArgs a, bool sp, hipStream_t s) {
   }
 }
 
-hipError_t launch_packed_gemm(const PackedGemmArgs& a, PackedTile tile, bool sp, hipStream_t s, hipEvent_t done) {
+hipError_t launch_packed_gemm(const PackedGemmArgs& a, PackedTile tile, int products, hipStream_t s, hipEvent_t done) {
+  using T = PackedTile;
   if (a.Hp) {
     if (a.splits != 1) return hipErrorInvalidValue;
-    if (sp) {
-      switch (tile) {
-        case PackedTile::k256x128: return launch_shape<256, 128, 4, 2, 3, true, true>(a, s, done);
-        case PackedTile::k128x128: return launch_shape<128, 128, 2, 2, 4, true, true>(a, s, done);
-        case PackedTile::k128x64: return launch_shape<128, 64, 2, 2, 3, true, true>(a, s, done);
-        default: return hipErrorInvalidValue;
-      }
+    if (products == 3) {
+      if (tile == T::k256x128) return launch_shape<256, 128, 4, 2, 3, 3, true>(a, s, done);
+      if (tile == T::k128x128) return launch_shape<128, 128, 2, 2, 4, 3, true>(a, s, done);
+      if (tile == T::k128x64) return launch_shape<128, 64, 2, 2, 3, 3, true>(a, s, done);
+    } else if (products == 1) {
+      if (tile == T::k256x256) return launch_shape<256, 256, 2, 4, 4, 1, true>(a, s, done);
+      if (tile == T::k128x128) return launch_shape<128, 128, 2, 2, 4, 1, true>(a, s, done);
     }
-    switch (tile) {
-      case PackedTile::k256x256: return launch_shape<256, 256, 2, 4, 4, false, true>(a, s, done);
-      case PackedTile::k128x128: return launch_shape<128, 128, 2, 2, 4, false, true>(a, s, done);
-      default: return hipErrorInvalidValue;
-    }
+    return hipErrorInvalidValue;
   }
-  if (sp) {
-    switch (tile) {
-      case PackedTile::k256x128: return launch_shape<256, 128, 4, 2, 3, true>(a, s, done);
-      case PackedTile::k192x128: return launch_shape<192, 128, 2, 2, 4, true>(a, s, done);
-      case PackedTile::k128x128: return launch_shape<128, 128, 2, 2, 4, true>(a, s, done);
-      case PackedTile::k128x64: return launch_shape<128, 64, 2, 2, 3, true>(a, s, done);
-      default: return hipErrorInvalidValue;
-    }
+  if (products == 3) {
+    if (tile == T::k256x128) return launch_shape<256, 128, 4, 2, 3, 3>(a, s, done);
+    if (tile == T::k192x128) return launch_shape<192, 128, 2, 2, 4, 3>(a, s, done);
+    if (tile == T::k128x128) return launch_shape<128, 128, 2, 2, 4, 3>(a, s, done);
+    if (tile == T::k128x64) return launch_shape<128, 64, 2, 2, 3, 3>(a, s, done);
+  } else if (products == 2) {
+    if (tile == T::k256x128) return launch_shape<256, 128, 4, 2, 4, 2>(a, s, done);
+    if (tile == T::k192x128) return launch_shape<192, 128, 2, 2, 4, 2>(a, s, done);
+    if (tile == T::k128x128) return launch_shape<128, 128, 2, 2, 3, 2>(a, s, done);
+    if (tile == T::k128x64) return launch_shape<128, 64, 2, 2, 4, 2>(a, s, done);
+  } else if (products == 1) {
+    if (tile == T::k256x256) return launch_shape<256, 256, 2, 4, 4, 1>(a, s, done);
+    if (tile == T::k192x128) return launch_shape<192, 128, 2, 2, 4, 1>(a, s, done);
+    if (tile == T::k128x128) return launch_shape<128, 128, 2, 2, 4, 1>(a, s, done);
   }
-  switch (tile) {
-    case PackedTile::k256x256: return launch_shape<256, 256, 2, 4, 4, false>(a, s, done);
-    case PackedTile::k192x128: return launch_shape<192, 128, 2, 2, 4, false>(a, s, done);
-    case PackedTile::k128x128: return launch_shape<128, 128, 2, 2, 4, false>(a, s, done);
-    default: return hipErrorInvalidValue;
-  }
+  return hipErrorInvalidValue;
 }
 
-PackedPlan plan_packed(int m, int rows, int K, bool sp, bool pairs, int splits) {
+PackedPlan plan_packed(int m, int rows, int K, int products, bool pairs, int splits) {
   // The fullest CU's tiles times the stages of one, at the measured time of a stage (32 k; us, on
   // 961 x 4864 x 896, 961 x 896 x 4864, 4096^3 and 2048 x 14336 x 4096), plus the bytes of the
   // outputs and, for K slices, of the partial tiles and their reduce at 4 TB/s and its launch.
@@ -461,8 +461,10 @@ PackedPlan plan_packed(int m, int rows, int K, bool sp, bool pairs, int splits) 
                              {PackedTile::k128x128, 128, 128, 0.222}};
   static const Shape f32[] = {{PackedTile::k256x128, 256, 128, 0.95}, {PackedTile::k192x128, 192, 128, 0.80},
                               {PackedTile::k128x128, 128, 128, 0.55}, {PackedTile::k128x64, 128, 64, 0.36}};
-  const Shape* sh = sp ? f32 : bf;
-  const int ns = sp ? 4 : 3, steps = (K + 31) / 32;
+  static const Shape f32b[] = {{PackedTile::k256x128, 256, 128, 0.66}, {PackedTile::k192x128, 192, 128, 0.55},
+                               {PackedTile::k128x128, 128, 128, 0.38}, {PackedTile::k128x64, 128, 64, 0.26}};
+  const Shape* sh = products == 3 ? f32 : products == 2 ? f32b : bf;
+  const int ns = products > 1 ? 4 : 3, steps = (K + 31) / 32;
   const double out_us = (double)m * rows * 4 / 4e6;
   const int first = splits ? splits : 1, last = splits ? splits : pairs ? 1 : 8;
   PackedPlan best;

@@ -90,6 +90,30 @@ def test_dense_k_remainders(t, monkeypatch):
         q.close()
 
 
+def test_bf16_weights_have_no_remainder():
+    """BF16 weights in f32 mode are one plane: an infinite weight meets both parts of x (of one sign here) and
+    stays infinite, as in the unpacked GEMM; the others' outputs are the unpacked GEMM's to 32-bit sums."""
+    m, n, rows = 300, 512, 260
+    rng = np.random.default_rng(13)
+    w = rng.standard_normal((m, n)).astype(np.float32)
+    w[5, 17], w[40, 0] = np.inf, -np.inf
+    q = rehip.QMat.from_bytes(rehip.BF16, (w.view(np.uint32) >> 16).astype(np.uint16).view(np.uint8).reshape(-1), m, n)
+    x = rng.standard_normal((rows, n)).astype(np.float32)
+    x[:, [0, 17]] = 1 + 2.0 ** -10
+    got = []
+    for knob in ("2", "0"):
+        with pytest.MonkeyPatch.context() as mp:
+            mp.setenv("REHIP_GEMM_PACKED", knob)
+            got.append(run(q, B.from_array(x), rows, m, rehip.MODE_F32).reshape(rows, m))
+    assert np.all(got[0][:, 5] == np.inf) and np.all(got[0][:, 40] == -np.inf)
+    assert np.array_equal(np.isfinite(got[0]), np.isfinite(got[1]))
+    fine = np.isfinite(w).all(1)
+    absd = np.abs(x).astype(np.float64) @ np.abs(w[fine]).astype(np.float64).T
+    # two products per pair, so 2 n additions of 2^-24 in either order
+    assert np.all(np.abs(got[0][:, fine] - got[1][:, fine]) <= 2 * 2 * n * 2.0 ** -24 * absd)
+    q.close()
+
+
 def test_operands_in_pieces():
     """Operands beyond the no-allocation scratch are packed and multiplied in pieces: the same bits."""
     t, m, n, rows = rehip.Q4_0, 700, 16384, 600
