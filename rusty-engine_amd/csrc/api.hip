@@ -559,24 +559,37 @@ struct PackedCall {
   static size_t pad(size_t r) { return (r + kPackedRows - 1) / kPackedRows * kPackedRows; }
 };
 
-// Whether packed operands beat decoding in the GEMM, by shape (measured over K 256 .. 14336, m 128 ..
-// 14336 and 64 .. 2048 rows, back to back, us tiled / packed; Q4_K, Q5_0, Q6_K and F16 agree).
-// Packing decodes each weight and converts each activation once, but writes 2 bytes (f32 mode 4) per
-// element and costs a launch.
-//   Quantized weights, whatever the rows: not where the tiled GEMM runs unsplit as one round of
-//   workgroups over a short K (m x K 4864 x 896, 961 rows, bf16: 22.4 / 26.9; 14336 x 512, 512 rows:
-//   19.8 / 27.9; f32 2048 x 768, 961 rows: 21.1 / 25.3).
+// Whether packed operands beat decoding in the GEMM, by shape (measured back to back over K 512 .. 14336, m 64
+// .. 28672 and 64 .. 4096 rows; m x K, us tiled / packed). Packing decodes each weight and converts each
+// activation once, but writes 2 bytes (f32 mode 4) per element, reads them again and costs a launch. Of
+// the measured shapes that the rule packs, one in thirty is slower so, by at most a tenth or so.
+//   Quantized weights (Q4_K; Q5_0, Q6_K and Q8_0 agree), whatever the rows: not where the tiled GEMM runs
+//   unsplit as one round of workgroups over a short K (4864 x 896, 961 rows, bf16: 22.4 / 26.9; 14336 x 512, 512
+//   rows: 19.8 / 27.9; f32 2048 x 768, 961 rows: 21.1 / 25.3).
 //   bf16 mode: from 384 rows (4864 x 896, 512 rows: 26.5 / 18.8; 896 x 896: 17.2 / 13.7), from 192 if
-//   the product is large and K is not short (4096 x 14336, 192 rows: 106 / 68; 4096 x 4096: 36.0 /
-//   31.6; 896 x 896, 320 rows: 10.1 / 13.9).
-//   f32 mode: from 320 rows (4096 x 4096: 102 / 56), from 192 for matrices up to 5M weights (4864 x
-//   896: 25.3 / 23.5; 4096 x 14336, 256 rows: 131 / 186), from 96 up to 1.6M (896 x 896, 128 rows:
-//   19.7 / 13.1; 4864 x 896, 96 rows: 21.7 / 22.2).
-//   Dense weights (F16, bf16 / f32 mode): from 256 rows and 256 weight rows (896 x 896: 14.3 / 13.5;
-//   128 x 896, 1024 rows: 10.1 / 12.9), from 128 rows for 4M weights and more (4864 x 896: 21.1 /
-//   17.3, 23.6 / 22.8; 2048 x 768, f32: 14.6 / 15.9).
-bool packed_pays(bool dense, size_t m, size_t K, size_t rows, bool sp) {
-  if (dense) return (rows >= 256 && m >= 256) || (rows >= 128 && m * K >= 4000000);
+//   the product is large and K is not short (4096 x 14336, 192 rows: 102 / 64; 4096 x 4096: 35 / 28; 896 x 896,
+//   320 rows: 10.1 / 13.9). Few weight rows do not pay for packing many activations (128 x 14336, 961 rows:
+//   23.7 / 33.6; 128 x 4096: 16.3 / 18.8, 384 rows 13.8 / 14.3; 256 x 4096, 961 rows: 20.5 / 19.6, 2048 rows 21.7 / 24.5;
+//   512 x 8192, 1024 rows: 0.87x).
+//   f32 mode: from 320 rows (4096 x 14336: 296 / 179, 256 rows 119 / 149; 4096 x 4096: 96 / 54), from 192 for
+//   matrices up to 5M weights (4864 x 896: 25.3 / 23.5), from 96 up to 1.6M (896 x 896, 128 rows: 19.7 / 13.1;
+//   4864 x 896, 96 rows: 21.7 / 22.2). Not for few weight rows over a long K (128 x 14336, 961 rows: 30 / 42; 64 x
+//   4096: 17.8 / 22.1; 512 x 4096, 192 rows: 0.94x).
+//   Dense weights: from 256 rows and 2.7e8 products (F16, bf16 / f32 mode, 896 x 896, 384 rows: 1.4x / 1.17x, 256
+//   rows 0.99x / 0.94x); F32 weights in f32 mode, whose tiled GEMM has least to prepare, from 384 rows and 6e8
+//   (14336 x 4096, 256 rows: 154 / 184, 512 rows 279 / 231). Fewer than 768 weight rows need more rows
+//   (512 x 4096, 256 rows: 0.75x .. 0.95x; 256 x 4096, 1024 rows: 1.12x). Not F32 and BF16 over a short K
+//   where the tiled GEMM runs 512 .. 768 workgroups, unsplit (4096 x 512, 512 rows: 0.73x .. 0.91x).
+bool packed_pays(uint32_t type, size_t m, size_t K, size_t rows, bool sp) {
+  if (dense_type(type)) {
+    const bool f32w = type == 0 && sp;
+    if (rows < (f32w ? 384 : 256) || (double)m * K * rows < (f32w ? 6e8 : 2.7e8)) return false;
+    const size_t tiles = ((m + 63) / 64) * ((rows + 63) / 64);
+    if (type != 1 && K <= 1024 && tiles >= 512 && tiles <= 768) return false;
+    if (m >= 768) return true;
+    if (m >= 384 && !f32w && (K < 8 * m || rows >= 384)) return true;
+    return m >= 192 && rows >= (f32w ? 1024 : 512) && rows * K >= 6000000;
+  }
   const GemmPlan pl = plan_gemm((int)m, (int)rows, (int)K, sp ? kGemmModeSplit : RE_MODE_BF16);
   if (pl.splits == 1 && K <= 1024 && pl.tile != GemmTile::k128x128) {
     const size_t bm = pl.tile == GemmTile::k64x64 ? 64 : 128;
@@ -585,7 +598,12 @@ bool packed_pays(bool dense, size_t m, size_t K, size_t rows, bool sp) {
     // one round: a 64 x 64 tile's stages let two workgroups share a CU
     if (tiles <= (bm == 64 ? 512u : 256u) && tiles > (bm == 64 ? 256u : 128u)) return false;
   }
-  if (sp) return rows >= 320 || (rows >= 192 && m * K <= 5000000) || (rows >= 96 && m * K <= 1600000);
+  const size_t x = rows * K;                      // activations to pack
+  if (sp) {
+    if (m < 640 && ((K >= 3072 && K >= 16 * m) || (K >= 4096 && x < 2600000) || (m <= 128 && x > 4100000))) return false;
+    return rows >= 320 || (rows >= 192 && m * K <= 5000000) || (rows >= 96 && m * K <= 1600000);
+  }
+  if (m < 768 && x > (m <= 128 ? 1500000u : 5000000u)) return false;
   return rows >= 384 || (rows >= 192 && K >= 1024 && (double)m * K * rows >= 3e9);
 }
 
@@ -597,7 +615,7 @@ bool packed_call(uint32_t type, const void* W, size_t m, size_t K, size_t KB, co
   const bool sp = mode == RE_MODE_F32;
   const size_t knob = env_size("REHIP_GEMM_PACKED", 1);
   if (knob == 0 || rows < 2 || !aligned16(d_x)) return false;
-  if (knob != 2 && !packed_pays(dense_type(type), m, K, rows, sp)) return false;
+  if (knob != 2 && !packed_pays(type, m, K, rows, sp)) return false;
   if (env_size("REHIP_GEMM_SP", 1) == 0 || env_size("REHIP_GEMM_TILE", 0)) return false;
   c->type = type;
   c->W = W;

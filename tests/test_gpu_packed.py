@@ -77,6 +77,25 @@ def test_planned_tiles(mode, m, n, rows):
     q.close()
 
 
+@pytest.mark.parametrize("t,m,n,rows,mode", [(rehip.Q4_K, 128, 8192, 512, rehip.MODE_BF16),
+                                             (rehip.Q4_K, 128, 8192, 512, rehip.MODE_F32),
+                                             (rehip.F16, 256, 2048, 256, rehip.MODE_BF16),
+                                             (rehip.F32, 512, 4096, 384, rehip.MODE_F32)])
+def test_small_products_are_not_packed(t, m, n, rows, mode):
+    """Shapes where packing costs more than it gives run the unpacked GEMM: its bits (other K slices than the
+    packed one's)."""
+    rng = np.random.default_rng(m + rows)
+    q = rehip.QMat.from_bytes(t, weights(rng, t, m, n), m, n)
+    dx = B.from_array(synth.activations(rng, rows, n))
+    got = {}
+    for knob in ("0", "1", "2"):
+        with pytest.MonkeyPatch.context() as mp:
+            mp.setenv("REHIP_GEMM_PACKED", knob)
+            got[knob] = run(q, dx, rows, m, mode)
+    assert np.array_equal(got["1"], got["0"]) and not np.array_equal(got["2"], got["0"])
+    q.close()
+
+
 @pytest.mark.parametrize("t", [rehip.F16, rehip.F32])
 def test_dense_k_remainders(t, monkeypatch):
     """Dense rows need whole 8-element units only: K that ends inside a fragment and a stage."""
