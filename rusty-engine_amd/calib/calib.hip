@@ -3,6 +3,7 @@
 // dependency-free MFMA stream and an empty kernel. bench.py times them with HIP
 // events to measure what this GPU reaches (HBM read bandwidth with the default and the
 // nontemporal cache policy, bf16 MFMA throughput, the per-launch floor of a graph of kernels).
+// cal_buffer_range answers a test's question about the card's range check of raw buffer loads.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -96,6 +97,27 @@ __global__ __launch_bounds__(256) void mfma_stream_kernel(float* out, int iters)
   if (lane == 0) out[blockIdx.x * 4 + (threadIdx.x >> 6)] = s;
 }
 
+// What raw buffer loads return through a resource of `records` bytes over p, lane l at vector offset 4 l (b32) or
+// 16 l (b128, and the copy into LDS) and scalar offset soffset. out: 4 x 64 words (the b32 word, the first
+// and the last word of the b128, the first word copied).
+__global__ __launch_bounds__(64) void buffer_range_kernel(const uint32_t* p, uint32_t records, int soffset, uint32_t* out) {
+  __shared__ __attribute__((aligned(16))) uint32_t copy[64 * 4];
+  typedef __attribute__((address_space(3))) void lds_void_t;
+  const int l = threadIdx.x;
+  const __amdgpu_buffer_rsrc_t r =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(p), (short)0, (int)records, 0x00020000);
+  for (int i = 0; i < 4; ++i) copy[4 * l + i] = ~0u;
+  __syncthreads();
+  const i32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(r, 16 * l, soffset, 0);
+  out[l] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r, 4 * l, soffset, 0);
+  out[64 + l] = (uint32_t)v[0];
+  out[128 + l] = (uint32_t)v[3];
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void_t*)copy, 16, 16 * l, soffset, 0, 0);
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  out[192 + l] = copy[4 * l];
+}
+
 __global__ void empty_kernel() {}
 
 }  // namespace
@@ -128,6 +150,14 @@ int cal_stream_read_chunk(const void* p, uint64_t bytes, int nontemporal, uint32
 // grid workgroups of 4 waves; out: grid * 4 floats; FLOP = grid * 4 * iters * 8 * 32768
 int cal_mfma(float* out, int grid, int iters, void* stream) {
   hipLaunchKernelGGL(mfma_stream_kernel, dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, out, iters);
+  return (int)hipGetLastError();
+}
+
+// p: `bytes` bytes that hold the records and every address the offsets could form; out: 256 words
+int cal_buffer_range(const void* p, uint64_t bytes, uint32_t records, uint32_t soffset, uint32_t* out, void* stream) {
+  if (records > bytes || (uint64_t)soffset + 64 * 16 > bytes) return (int)hipErrorInvalidValue;
+  hipLaunchKernelGGL(buffer_range_kernel, dim3(1), dim3(64), 0, (hipStream_t)stream, (const uint32_t*)p, records,
+                     (int)soffset, out);
   return (int)hipGetLastError();
 }
 

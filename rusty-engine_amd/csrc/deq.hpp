@@ -70,7 +70,10 @@ __device__ __forceinline__ uint4 ld16(const uint8_t* p) { return *reinterpret_ca
 
 // Raw buffer loads through a resource covering a whole matrix (or all experts): byte offsets are
 // 32-bit and a read past num_records returns zero, so padding rows/columns need no branches
-// (zero bytes decode to zero weights for every type: every scale is then 0).
+// (zero bytes decode to zero weights for every type: every scale is then 0). On this card the scalar
+// offset counts in the check like the vector one, also where it alone is past the end, and so it does in
+// copies into LDS; kernels here rely on that for rows and blocks past the end (the compiler's intrinsics
+// only promise it for the vector offset: tests/test_gpu_buffer_range.py holds the card to it).
 typedef __attribute__((__vector_size__(4 * sizeof(int)))) int i32x4_t;
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, 0x00020000);

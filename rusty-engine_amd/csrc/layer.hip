@@ -765,7 +765,8 @@ __global__ __launch_bounds__(64 * kAttnMfmaWaves) void attention_mfma_kernel(
   const int limit = r < rows ? max(min(p0 + r, max_seq - 1), 0) : -1;
   const int lim_first = max(min(p0 + g0 / grp, max_seq - 1), 0);   // of the block's first vector
   // one per-lane offset plus a scalar row offset; the resources end with the last visible row, so
-  // rows past it are never read (zeros, which no vector sees)
+  // rows past it are never read (zeros, which no vector sees; the range check counts the scalar offset,
+  // see make_rsrc)
   const uint32_t row_b = (uint32_t)kv_dim * 4u, cache_b = (uint32_t)jmax * row_b + HD * 4u;
   const __amdgpu_buffer_rsrc_t kr = make_rsrc(kc + (size_t)kvh * HD, cache_b);
   const __amdgpu_buffer_rsrc_t vr = make_rsrc(vc + (size_t)kvh * HD, cache_b);
