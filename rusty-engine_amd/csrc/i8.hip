@@ -79,7 +79,9 @@ constexpr int kI8MagicBits = 0x4B400000;
 // block-major; weights load into registers kI8Ahead blocks ahead, at a scalar offset. No branch
 // inside a stage (a branch between an MFMA and the reads of its result, or between a load and its
 // use, makes the compiler wait for every outstanding load).
-// 4864 x 896, 961 rows, with the quantization: 34.8 -> 29.2 us (the three-operation fold alone 34.5).
+// 4864 x 896, 961 rows, with the quantization: 34.8 -> 29.2 us (the three-operation fold alone 34.5); rows of
+// 4864: 1.5-1.7 times as fast; rows of 512 (four stages) 0.5 us slower, 7.2 -> 7.7, for the first stage's way
+// through LDS.
 // A scale that is not finite has no exact bias and leaves NaN: such rows are folded again at the end.
 __global__ __launch_bounds__(256, 4) void q8_i8_gemm_kernel(const uint8_t* __restrict__ W, const float* __restrict__ xs,
                                                          const int8_t* __restrict__ xq, float* __restrict__ y, int m,
@@ -96,7 +98,7 @@ __global__ __launch_bounds__(256, 4) void q8_i8_gemm_kernel(const uint8_t* __res
   const int tile = min(2 * (int)blockIdx.x + (wave >> 1), tiles - 1);   // past the last: computed, not stored
   const int h = lane >> 5, c = lane & 31;
   const int trow = (wave & 1) * 32 + c;                 // weight row inside the tile
-  // the tile's slabs and the group's activation rows, each below 2 GiB (n <= 2^24)
+  // the tile's slabs and the group's activation rows, each below 2 GiB (a matrix has at most 2^24 columns)
   const __amdgpu_buffer_rsrc_t wr = make_rsrc(W + (size_t)tile * nb * SLAB, (uint32_t)nb * SLAB);
   const __amdgpu_buffer_rsrc_t ar = make_rsrc(xq + (size_t)r0 * n, (uint32_t)min(32, rows - r0) * (uint32_t)n);
   const int wo = h * (64 * 16) + trow * 16, wdo = 2 * (64 * 16) + trow * 2;
@@ -394,9 +396,8 @@ hipError_t launch_q8_i8_gemm(const uint8_t* W, int tiles, const float* xs, const
     return hipGetLastError();
   }
   const unsigned rgroups = (unsigned)((rows + 31) / 32);
-  // long rows over few output tiles: split each tile's fold over the waves of a workgroup (and rows past
-  // the 32-bit offsets of the other kernel)
-  if ((n >> 5) >= 64 && ((size_t)tiles * 2 * rgroups < 512 || n > (1 << 24))) {
+  // long rows over few output tiles: split each tile's fold over the waves of a workgroup
+  if ((n >> 5) >= 64 && (size_t)tiles * 2 * rgroups < 512) {
     const size_t lds = (size_t)min(n >> 5, kI8Chunk) * 32 * sizeof(float);
     hipLaunchKernelGGL(q8_i8_gemm_seg_kernel, dim3((unsigned)tiles * 2, rgroups), dim3(64 * kSegWaves), lds, s, W,
                        xs, xq, y, m, n, rows);
