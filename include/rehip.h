@@ -91,7 +91,9 @@ int re_qmat_matmul(re_qmat *q, const float *x, size_t rows, float *y, int mode);
 /* Device-pointer variants; `stream` is a hipStream_t (NULL = default stream). re_qmat_matmul_dev
  * allocates on first use: up to 32 MiB per matrix for K-split partial tiles and, for the calls of many
  * rows that run on packed bf16 operands, workspaces shared by all matrices of a GPU (at most 4 of
- * 64 .. 512 MiB, ordered between streams by events, freed with the last matrix). */
+ * 64 .. 512 MiB, ordered between streams by events, freed with the last matrix). Under stream capture, or
+ * without memory for a workspace, such calls run the unpacked GEMM: results that differ by the order of
+ * the sums. */
 int re_qmat_matvec_dev(re_qmat *q, const float *d_x, float *d_y, void *stream);
 int re_qmat_matmul_dev(re_qmat *q, const float *d_x, size_t rows, float *d_y, int mode,
                        void *stream);
@@ -102,12 +104,12 @@ int re_qmat_matmul_dev(re_qmat *q, const float *d_x, size_t rows, float *d_y, in
  * and results as re_qmat_matmul_dev, except where packed operands exceed the scratch: they are then packed
  * and multiplied in pieces (the same results) or, if the pieces would be too small to fill the GPU, the
  * unpacked GEMM runs (results that differ by the order of the sums). A plan whose partials exceed the
- * scratch fails with RE_ERR_SIZE (the planned splits of every shape fit: the planner caps partial tiles at
- * 32 MiB). The scratch is shared by every call on a GPU. Outside stream capture, a call first waits for the launches of the
- * previous call on that GPU (an event set up once per device), so calls from several streams or threads
- * stay ordered. Inside stream capture no ordering is added: replays of captured graphs that use the
- * scratch must not overlap in time. Those are the graphs of quantized calls with K slices; dense weights
- * and single-slice calls are captured without the scratch, as the unpacked GEMM. */
+ * scratch fails with RE_ERR_SIZE (the planned splits of every shape fit: the planner caps partial tiles
+ * at 32 MiB). The scratch is shared by every call on a GPU. Outside stream capture, a call first waits for
+ * the launches of the previous call on that GPU (an event set up once per device), so calls from several
+ * streams or threads stay ordered. Inside stream capture no ordering is added: replays of captured graphs
+ * that use the scratch must not overlap in time. Those are the graphs of quantized calls with K slices;
+ * dense weights and single-slice calls are captured as the unpacked GEMM, without the scratch. */
 int re_qmat_matmul_noalloc_dev(re_qmat *q, const float *d_x, size_t rows, float *d_y, int mode, void *stream);
 /* Dequantize the resident weights to d_out[m x n] f32, bit-exact with quant::dequant. */
 int re_qmat_dequant_dev(re_qmat *q, float *d_out, void *stream);
