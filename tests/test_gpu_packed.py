@@ -6,6 +6,8 @@ Bounds per output, relative to sum |w x|: bf16 has 8 significant bits, so a roun
 2^-8 and a bf16-mode product by 2^-7 + 2^-16; in f32 mode a remainder is at most 2^-8 of its value and
 its rounding leaves 2^-16, so a product is off by 2^-16 for either operand and 2^-16 for the dropped
 lo x lo (and 2^-32). The f32 sums add K roundings of 2^-24, whatever the MFMAs' order."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -222,6 +224,38 @@ def test_streams_come_and_go():
         again.destroy()
     q.close()
     big.close()
+
+
+def test_results_reach_the_host():
+    """The workspace's event carries no system-scope release: outputs still reach the host by a copy on the
+    call's stream, by one on another stream after a synchronize, and written into pinned host memory."""
+    m, n, rows = 896, 4864, 400
+    rng = np.random.default_rng(9)
+    q = rehip.QMat.from_bytes(rehip.Q6_K, weights(rng, rehip.Q6_K, m, n), m, n)
+    dx = [B.from_array(synth.activations(rng, rows, n)) for _ in range(2)]
+    want = [run(q, x, rows, m, rehip.MODE_BF16) for x in dx]
+    H, y, size = hip.hip(), B(rows * m * 4), C.c_size_t(rows * m * 4)
+    pinned, on_device = C.c_void_p(), C.c_void_p()
+    hip.check(H.hipHostMalloc(C.byref(pinned), size, 0))
+    hip.check(H.hipHostGetDevicePointer(C.byref(on_device), pinned, 0))
+    got = np.ctypeslib.as_array(C.cast(pinned, C.POINTER(C.c_float)), (rows * m,))
+    s, other = hip.Stream(), hip.Stream()
+    for i in range(30):
+        x, w = dx[i % 2], want[i % 2]
+        for way in (s, other, None):
+            got[:] = -1
+            q.matmul_dev(x, rows, y if way else on_device.value, rehip.MODE_BF16, stream=s)
+            if way is not s:
+                s.synchronize()
+            if way:
+                hip.check(H.hipMemcpyAsync(pinned, C.c_void_p(y.ptr), size, 2, C.c_void_p(way.handle)))
+                way.synchronize()
+            assert np.array_equal(got, w), (i, way)
+    del got
+    hip.check(H.hipHostFree(pinned))
+    for o in (s, other):
+        o.destroy()
+    q.close()
 
 
 def test_capture_after_eager_call_keeps_its_slices():
