@@ -7,6 +7,7 @@ Bounds per output, relative to sum |w x|: bf16 has 8 significant bits, so a roun
 its rounding leaves 2^-16, so a product is off by 2^-16 for either operand and 2^-16 for the dropped
 lo x lo (and 2^-32). The f32 sums add K roundings of 2^-24, whatever the MFMAs' order."""
 import ctypes as C
+import threading
 
 import numpy as np
 import pytest
@@ -224,6 +225,41 @@ def test_streams_come_and_go():
         again.destroy()
     q.close()
     big.close()
+
+
+def test_threads():
+    """More threads than workspaces, each with its own matrix and stream (two of them with the per-thread
+    default stream, one handle for two streams): every call gets its own product."""
+    m, n, rows = 640, 1024, 400
+    rng = np.random.default_rng(10)
+    jobs = []
+    for i in range(6):
+        q = rehip.QMat.from_bytes(rehip.Q8_0, weights(rng, rehip.Q8_0, m, n), m, n)
+        x = B.from_array(synth.activations(rng, rows, n))
+        jobs.append((q, x, run(q, x, rows, m, rehip.MODE_F32), [B(rows * m * 4) for _ in range(20)]))
+    errors = []
+
+    def work(i):
+        try:
+            q, x, _, ys = jobs[i]
+            s = hip.Stream() if i < 4 else None
+            for y in ys:                       # (hipStreamPerThread is the handle 2)
+                q.matmul_dev(x, rows, y, rehip.MODE_F32, stream=s or 2)
+            if s:
+                s.destroy()
+        except Exception as e:                 # noqa: BLE001
+            errors.append(e)
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(jobs))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    hip.synchronize()
+    assert not errors
+    for q, _, want, ys in jobs:
+        for y in ys:
+            assert np.array_equal(y.download(np.float32, rows * m), want)
+        q.close()
 
 
 def test_results_reach_the_host():
