@@ -79,9 +79,10 @@ constexpr int kI8MagicBits = 0x4B400000;
 // block-major; weights load into registers kI8Ahead blocks ahead, at a scalar offset. No branch
 // inside a stage (a branch between an MFMA and the reads of its result, or between a load and its
 // use, makes the compiler wait for every outstanding load).
-// 4864 x 896, 961 rows, with the quantization: 34.8 -> 29.2 us (the three-operation fold alone 34.5); rows of
-// 4864: 1.5-1.7 times as fast; rows of 512 (four stages) 0.5 us slower, 7.2 -> 7.7, for the first stage's way
-// through LDS.
+// The first stage's activations and scales are loaded together (one after the other, rows of 256 and 512 were
+// 0.5-0.9 us slower than read straight from the rows). 4864 x 896, 961 rows: 32.4 -> 23.1 us, rows of 4864 154
+// -> 107 us, rows of 256 4.9 -> 4.9 at 32 rows (the three-operation fold alone: 4864 x 896 34.8 -> 34.5 with the
+// quantization).
 // A scale that is not finite has no exact bias and leaves NaN: such rows are folded again at the end.
 __global__ __launch_bounds__(256, 4) void q8_i8_gemm_kernel(const uint8_t* __restrict__ W, const float* __restrict__ xs,
                                                          const int8_t* __restrict__ xq, float* __restrict__ y, int m,
@@ -117,9 +118,20 @@ __global__ __launch_bounds__(256, 4) void q8_i8_gemm_kernel(const uint8_t* __res
     Bw[j] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wr, wo, kn * (int)SLAB, 0));
     D[j] = __builtin_amdgcn_raw_buffer_load_b16(wr, wdo, kn * (int)SLAB, 0);
   };
+  // scales of four of this thread's blocks of a row, every eighth from k0 of the chunk at kb0
+  const int st = threadIdx.x & 31, sk = threadIdx.x >> 5;
+  const float* srow = xs + (size_t)min(r0 + st, rows - 1) * nb;
+  float sv[4];
+  auto load_s = [&](const int kb0, const int kc, const int k0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) sv[u] = srow[kb0 + min(k0 + 8 * u, kc - 1)];
+  };
+  // the first stage's activations and scales go out together, ahead of the weights: one memory round trip
   uint4 xv = load_x(0);
+  load_s(0, min(kI8Chunk, nb), sk);
 #pragma unroll
   for (int j = 0; j < kI8Ahead; ++j) load(j, j);
+  __builtin_amdgcn_sched_barrier(0);
   float s[16];
 #pragma unroll
   for (int i = 0; i < 16; ++i) s[i] = 0.0f;
@@ -149,22 +161,18 @@ __global__ __launch_bounds__(256, 4) void q8_i8_gemm_kernel(const uint8_t* __res
     __builtin_amdgcn_sched_barrier(0);   // else every refill moves ahead of the stage's first wait
   };
 
-  const int st = threadIdx.x & 31, sk = threadIdx.x >> 5;   // staging of scales: row, first block
-  const float* srow = xs + (size_t)min(r0 + st, rows - 1) * nb;
   xb[0][xd] = xv;
   xv = load_x(1);
   int buf = 0;
   for (int kb0 = 0; kb0 < nb; kb0 += kI8Chunk) {
     const int kc = min(kI8Chunk, nb - kb0);
     if (kb0) __syncthreads();
-    // scales of 32 activation rows x kc blocks -> dxs[block][row]; loads issued 4 at a time
+    // scales of 32 activation rows x kc blocks -> dxs[block][row]
     for (int k0 = sk; k0 < kc; k0 += 8 * 4) {
-      float v[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) v[u] = srow[kb0 + min(k0 + 8 * u, kc - 1)];
+      if (kb0 || k0 != sk) load_s(kb0, kc, k0);
 #pragma unroll
       for (int u = 0; u < 4; ++u)
-        if (k0 + 8 * u < kc) dxs[k0 + 8 * u][st] = v[u];
+        if (k0 + 8 * u < kc) dxs[k0 + 8 * u][st] = sv[u];
     }
     const int full = kc & ~(kI8Ahead - 1);
 #pragma unroll 1
