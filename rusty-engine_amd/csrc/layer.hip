@@ -875,48 +875,57 @@ __global__ __launch_bounds__(64 * kAttnMfmaWaves) void attention_mfma_kernel(
         for (int i = 0; i < 16; ++i) o[b][i] = __builtin_fmaf(o[b][i], alpha, p * vj[32 * b + attn_key_of(i, 0)]);
     }
   }
-  // wave partials: O^T register i of block b is dim 32 b + 8(i/4) + 4h + i%4 of vector vl
-  l += __shfl_xor(l, 32, 64);
+  // wave partials: O^T register i of block b is dim 32 b + 8(i/4) + 4h + i%4 of vector vl. Up to W / 2 key
+  // blocks leave the upper half of the waves without any, and their partials out of the combine.
+  const bool half = nkb <= W / 2;
+  if (w < W / 2 || !half) {
+    l += __shfl_xor(l, 32, 64);
 #pragma unroll
-  for (int b = 0; b < NB; ++b)
+    for (int b = 0; b < NB; ++b)
 #pragma unroll
-    for (int i = 0; i < 16; i += 4)
-      *reinterpret_cast<float4*>(&Os[w][vl][32 * b + attn_key_of(i, h)]) =
-          make_float4(o[b][i], o[b][i + 1], o[b][i + 2], o[b][i + 3]);
-  if (h == 0) {
-    Ms[w][vl] = m;
-    Ls[w][vl] = l;
+      for (int i = 0; i < 16; i += 4)
+        *reinterpret_cast<float4*>(&Os[w][vl][32 * b + attn_key_of(i, h)]) =
+            make_float4(o[b][i], o[b][i + 1], o[b][i + 2], o[b][i + 3]);
+    if (h == 0) {
+      Ms[w][vl] = m;
+      Ls[w][vl] = l;
+    }
   }
   __syncthreads();
   // combine: thread t -> vector t / 16, every 16th four dims from 4 (t % 16)
   const int v = threadIdx.x >> 4;
   const int gv = g0 + v, rv = gv / grp;
   if (rv >= rows) return;
-  float M = Ms[0][v];
-#pragma unroll
-  for (int k = 1; k < W; ++k) M = fmaxf(M, Ms[k][v]);
-  // (every score -inf: the differences are NaN and so is the row, as exp(x - max) gives it)
-  float f[W], tot = 0.0f;
-#pragma unroll
-  for (int k = 0; k < W; ++k) {
-    f[k] = expf(Ms[k][v] - M);
-    tot = __builtin_fmaf(Ls[k][v], f[k], tot);
-  }
-  const float inv = tot != 0.0f ? 1.0f / tot : 1.0f;
   float* out = ctx + ((size_t)rv * heads + kvh * grp + gv % grp) * HD;
+  auto combine = [&](auto waves) {
+    constexpr int C = decltype(waves)::value;
+    float M = Ms[0][v];
 #pragma unroll
-  for (int d = 4 * (threadIdx.x & 15); d < HD; d += 64) {
-    float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int k = 1; k < C; ++k) M = fmaxf(M, Ms[k][v]);
+    // (every score -inf: the differences are NaN and so is the row, as exp(x - max) gives it)
+    float f[C], tot = 0.0f;
 #pragma unroll
-    for (int k = 0; k < W; ++k) {
-      const float4 x = *reinterpret_cast<const float4*>(&Os[k][v][d]);
-      a.x = __builtin_fmaf(x.x, f[k], a.x);
-      a.y = __builtin_fmaf(x.y, f[k], a.y);
-      a.z = __builtin_fmaf(x.z, f[k], a.z);
-      a.w = __builtin_fmaf(x.w, f[k], a.w);
+    for (int k = 0; k < C; ++k) {
+      f[k] = expf(Ms[k][v] - M);
+      tot = __builtin_fmaf(Ls[k][v], f[k], tot);
     }
-    *reinterpret_cast<float4*>(out + d) = make_float4(a.x * inv, a.y * inv, a.z * inv, a.w * inv);
-  }
+    const float inv = tot != 0.0f ? 1.0f / tot : 1.0f;
+#pragma unroll
+    for (int d = 4 * (threadIdx.x & 15); d < HD; d += 64) {
+      float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+      for (int k = 0; k < C; ++k) {
+        const float4 x = *reinterpret_cast<const float4*>(&Os[k][v][d]);
+        a.x = __builtin_fmaf(x.x, f[k], a.x);
+        a.y = __builtin_fmaf(x.y, f[k], a.y);
+        a.z = __builtin_fmaf(x.z, f[k], a.z);
+        a.w = __builtin_fmaf(x.w, f[k], a.w);
+      }
+      *reinterpret_cast<float4*>(out + d) = make_float4(a.x * inv, a.y * inv, a.z * inv, a.w * inv);
+    }
+  };
+  if (half) combine(std::integral_constant<int, W / 2>{});
+  else combine(std::integral_constant<int, W>{});
 }
 
 // q/k/v projection rows (strided; q|k|v may be one fused projection) plus their biases ->
